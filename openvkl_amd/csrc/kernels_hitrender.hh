@@ -26,84 +26,100 @@ VKL_DEV float dot3(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 // Opacity 0.6 per shaded hit takes the accumulated opacity past 0.99 after
 // 6 hits (binary32: 0.6, 0.84, 0.936, 0.9744, 0.98976, 0.995904), so a ray
 // shades at most this many hits.
-constexpr int kMaxShadedHits = 8;
+constexpr int kMaxShadedHits = 6;
+
+// Lanes without a running query that let a wavefront stop for its shading.
+constexpr uint32_t kShadeVote = 16;
 
 // Two phases per ray, in the reference's order of results: first the
 // primary ray's hits that will be shaded (the compositing opacity does not
-// depend on the shading, so their number is known in advance; they wait in
-// LDS), then each hit in order: gradient normal, shadow rays, compositing.
-// Primary and shadow queries share one hit-iterator state and one hitNext
-// call site (the hit iteration is inlined once), and no second state is
-// parked, so the state stays in registers.
-// Occupancy: on structuredRegular sources 5 waves per SIMD (128 VGPRs at
-// most, 60-104 bytes of spill) measured fastest on a 1080p frame of the
-// 512^3 volume: 23.2 ms against 24.8 at 4 waves, 29.5 at 3 and 26.6 at 6.
-// Other sources keep 3 waves (168 VGPRs instead of 204 at 2, 35 % faster).
-// Cubic filters keep the compiler's choice.
+// depend on the shading, so their number is known in advance), then each hit
+// in order: gradient normal, shadow rays, compositing. Primary and shadow
+// queries share one search state and one hitTick call site. The hits and the
+// shading state wait in LDS while a query runs: they are touched once per
+// query, and in registers they displaced the search's own state.
+//
+// Bound by instruction issue with part of the lanes idle: a 1080p frame of a
+// 300 x 260 x 340 float volume with two iso values 31-33 -> 21-22 ms against
+// nested loops per query (22 instead of 9 lanes active, 212 k instead of
+// 538 k vector instructions a wavefront). 3 waves per SIMD (168 VGPRs): 2
+// waves 30 ms; 4 and more spill the search's state, 40-80 ms. Shading when
+// 12 to 28 lanes wait measured the same; waiting for all 64 took 7 % longer.
 template <typename Src, int kFilter, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((
-    amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : (IsDenseSource<Src>::value ? 5 : 3))))
+    amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : 3)))
 void kHitRender(const IteratorContextView *__restrict__ cp, AttrView a,
                                                           HitRenderArgs m)
 {
-  __shared__ float hitT[kMaxShadedHits][kIterBlock], hitS[kMaxShadedHits][kIterBlock],
-      hitE[kMaxShadedHits][kIterBlock];
+  __shared__ float hitT[kMaxShadedHits][kIterBlock], hitS[kMaxShadedHits][kIterBlock], hitE[kIterBlock];
+  __shared__ float bisect[kBisWords * kHitLanes];
+  __shared__ float sN[3][kIterBlock], sCi[kIterBlock], sCo[kIterBlock], sIllum[kIterBlock], sRgba[4][kIterBlock];
   const uint32_t r = xcdBandBlock(blockIdx.x, gridDim.x) * kIterBlock + threadIdx.x;
   if (r >= m.numRays) return;
   const uint32_t lane          = threadIdx.x;
   const IteratorContextView &c = *cp;
   PointSampler<Src, kFilter> smp(c.sampler.grid, a, c.attributeIndex);
   smp.setTime(m.time);
-  const F3 o = {m.org[3 * r], m.org[3 * r + 1], m.org[3 * r + 2]};
-  const F3 d = {m.dir[3 * r], m.dir[3 * r + 1], m.dir[3 * r + 2]};
-  const F3 light0 = normalize3(F3{1.f, 1.f, 1.f}), light1 = normalize3(F3{1.f, 1.f, -1.f});
-  const F3 wi     = normalize3(F3{-1.f * d.x, -1.f * d.y, -1.f * d.z});
   const uint32_t maxShade = m.maxHits < (uint32_t)kMaxShadedHits ? m.maxHits : (uint32_t)kMaxShadedHits;
 
-  HitState st;
-  hitInit<hitDepthOf<Src>()>(c, st, o, d, rayRange(m.tRanges, r), m.time);
-  bool primary = true;
+  HitSearch st;
+  hitInit<hitDepthOf<Src>()>(c, st.h, F3{m.org[3 * r], m.org[3 * r + 1], m.org[3 * r + 2]},
+                             F3{m.dir[3 * r], m.dir[3 * r + 1], m.dir[3 * r + 2]}, rayRange(m.tRanges, r), m.time);
+  hitBegin(st, bisect + lane);
+#pragma unroll
+  for (int i = 0; i < 4; i++) sRgba[i][lane] = 0.f;
+  bool searching = maxShade > 0, done = false;
   uint32_t hits = 0, k = 0;
   float alphaP = 0.f;  // opacity after the hits collected so far
-  // the hit being shaded
-  F3 p = {0.f, 0.f, 0.f}, N = {0.f, 0.f, 0.f};
-  float ci = 0.f, co = 0.f, illum = 0.f;
-  int light = -1;  // next light to test; -1: hit k not started
-  float cr = 0.f, cg = 0.f, cb = 0.f, alpha = 0.f;
-  for (;;) {
-    if (primary && !(alphaP < 0.99f && hits < maxShade)) {
-      primary = false;
-    } else {
+  int light    = -2;   // next light to test; -1: hit k not started; -2: collecting the hits
+  int event    = 0;
+  while (!done) {
+    if (searching) {
       HitOut h;
-      const bool got = hitNext<decltype(smp), kQuery>(c, smp, st, h);
-      if (primary) {
-        if (got) {
+      event = hitTick<decltype(smp), kQuery>(c, smp, st, h);
+      if (event) {
+        searching = false;
+        if (light == -2 && event == 1) {
           hitT[hits][lane] = h.t;
           hitS[hits][lane] = h.sample;
-          hitE[hits][lane] = h.epsilon;
+          hitE[lane]       = h.epsilon;  // of every hit of a ray
           hits++;
-          alphaP = alphaP + (1.f - alphaP) * 0.6f;
-          continue;
+          alphaP    = alphaP + (1.f - alphaP) * 0.6f;
+          searching = alphaP < 0.99f && hits < maxShade;
         }
-        primary = false;
-      } else {
-        if (!got) illum += fabsf(co) * (light == 0 ? 1.f : 0.8f);
-        light++;
       }
+    }
+    // Lanes whose query has ended wait until several of them can go on
+    // together: the shading below costs more instructions than a tick.
+    const uint32_t busy = (uint32_t)__popcll(__ballot(searching));
+    const uint32_t idle = (uint32_t)__popcll(__ballot(!searching));
+    if (idle < kShadeVote && busy != 0) continue;
+    if (searching) continue;
+    const F3 light0 = normalize3(F3{1.f, 1.f, 1.f}), light1 = normalize3(F3{1.f, 1.f, -1.f});
+    const F3 o = {m.org[3 * r], m.org[3 * r + 1], m.org[3 * r + 2]};
+    const F3 d = {m.dir[3 * r], m.dir[3 * r + 1], m.dir[3 * r + 2]};
+    F3 p = {0.f, 0.f, 0.f}, N = {sN[0][lane], sN[1][lane], sN[2][lane]};
+    float ci = sCi[lane], co = sCo[lane], illum = sIllum[lane];
+    if (light == -2) {
+      light = -1;
+    } else {
+      if (event == 2) illum += fabsf(co) * (light == 0 ? 1.f : 0.8f);
+      light++;
     }
     // Advance the shading to the next shadow query, compositing every hit
     // whose lights are done.
     bool query = false;
     while (k < hits) {
+      const float t = hitT[k][lane];
+      p             = F3{o.x + t * d.x, o.y + t * d.y, o.z + t * d.z};
       if (light < 0) {  // start hit k
-        const float t = hitT[k][lane];
-        p             = F3{o.x + t * d.x, o.y + t * d.y, o.z + t * d.z};
-        const F3 q    = xfmPoint(c.sampler.grid.o2i, p);
-        F3 gi         = {0.f, 0.f, 0.f};
+        const F3 wi = normalize3(F3{-1.f * d.x, -1.f * d.y, -1.f * d.z});
+        const F3 q  = xfmPoint(c.sampler.grid.o2i, p);
+        F3 gi       = {0.f, 0.f, 0.f};
         if (c.sampler.gradientFilter == kFilterLinear)
           gi = gradientLinear(smp.src, q);
         else if (c.sampler.gradientFilter == kFilterCubic)
-          gi = gradientCubic(smp.src, q);
+          gi = gradientCubicBySlices(smp.src, q);
         N = normalize3(xfmNormal(c.sampler.grid.o2i, gi));
         if (isnan(N.x) || isnan(N.y) || isnan(N.z)) N = F3{0.f, 0.f, 0.f};
         ci = dot3(N, wi);
@@ -127,20 +143,26 @@ void kHitRender(const IteratorContextView *__restrict__ cp, AttrView a,
       }
       float albedo[4];
       tfSampleRgba(m.tf, m.tfSize, m.tfLo, m.tfHi, hitS[k][lane], albedo);
-      cr    = cr + (1.f - alpha) * illum * albedo[0];
-      cg    = cg + (1.f - alpha) * illum * albedo[1];
-      cb    = cb + (1.f - alpha) * illum * albedo[2];
-      alpha = alpha + (1.f - alpha) * 0.6f;
+      const float alpha = sRgba[3][lane];
+      sRgba[0][lane]    = sRgba[0][lane] + (1.f - alpha) * illum * albedo[0];
+      sRgba[1][lane]    = sRgba[1][lane] + (1.f - alpha) * illum * albedo[1];
+      sRgba[2][lane]    = sRgba[2][lane] + (1.f - alpha) * illum * albedo[2];
+      sRgba[3][lane]    = alpha + (1.f - alpha) * 0.6f;
       k++;
       light = -1;
     }
-    if (!query) break;
-    hitInit<hitDepthOf<Src>()>(c, st, p, light == 0 ? light0 : light1, Range1f{hitE[k][lane], vinf()}, m.time);
+    if (query) {
+      sN[0][lane] = N.x, sN[1][lane] = N.y, sN[2][lane] = N.z;
+      sCi[lane] = ci, sCo[lane] = co, sIllum[lane] = illum;
+      hitInit<hitDepthOf<Src>()>(c, st.h, p, light == 0 ? light0 : light1, Range1f{hitE[lane], vinf()}, m.time);
+      hitBegin(st, bisect + lane);
+      searching = true;
+    } else {
+      done = true;
+    }
   }
-  m.rgba[4 * r]     = cr;
-  m.rgba[4 * r + 1] = cg;
-  m.rgba[4 * r + 2] = cb;
-  m.rgba[4 * r + 3] = alpha;
+#pragma unroll
+  for (int i = 0; i < 4; i++) m.rgba[4 * r + i] = sRgba[i][lane];
   if (m.count) m.count[r] = hits;
 }
 

@@ -40,26 +40,34 @@ VKL_DEV void tfSampleRgba(const float *__restrict__ tf, uint32_t n, float lo, fl
 
 VKL_DEV float minf_(float a, float b) { return a < b ? a : b; }
 
-// Samples of an interval taken together (independent loads in flight): 4
-// for vdb sources, whose samples wait on dependent index and leaf loads; 1
-// for structuredRegular ones, whose coherent rays hit the caches and which
-// lose more to the extra registers than they gain.
-template <typename Src>
-constexpr int samplesAhead()
-{
-  return IsDenseSource<Src>::value ? 1 : 4;
-}
+// Samples of an interval that a vdb march takes together (independent loads
+// in flight): its samples wait on dependent index and leaf loads. Dense
+// marches take one: their coherent rays hit the caches, and they lose more to
+// the extra registers than they gain.
+constexpr int kSamplesAhead = 4;
+
+// Lanes of a vdb march that wait for an interval, times this, against the
+// lanes that have samples to take: below it the interval phase waits.
+constexpr uint32_t kMarchIntervalVote = 3;
 
 // rgba[4r..4r+3] = composited colour and accumulated opacity of ray r.
-// structuredRegular sources: 5 waves per SIMD (96 VGPRs instead of 126 at 4
-// waves; with the dense query alone a 12-byte spill, 128 bytes with both
-// queries) measured fastest on a 1080p frame of the 512^3 volume (6 waves:
-// 80 VGPRs and a 112-byte spill, 1-7 % slower); vdb sources keep the
-// compiler's choice (no spill), which with 4 samples in flight measured 14 %
-// faster on the 4096^3 vdb; cubic filters keep the compiler's choice.
+//
+// vdb sources: bound by dependent loads and by lanes that wait for each
+// other, so the wavefront runs one loop in which the lanes whose interval is
+// used up visit the next voxel and the others take their next samples. 2^18
+// rays through a 1024^3 shell, camera / random: 6.26 / 6.23 -> 3.33 / 4.17 ms
+// at depth 2, 14.3 / 19.6 -> 5.3 / 5.9 ms at depth 3, against nested loops
+// per interval; 4 waves per SIMD (5 waves: 15-60 % slower; the compiler's 3
+// at depth 3: 9.2 ms for random rays).
+//
+// structuredRegular sources: bound by instruction issue on coherent rays,
+// whose lanes share voxel lines as long as they stay in step, which the
+// nested loops keep (one loop as above: 8.0-10.2 ms a 1080p frame of the
+// 512^3 volume against 4.9). 5 waves per SIMD: 94 VGPRs without spill at
+// depth 2, the default (4 waves the same, 6 waves 7 % slower).
 template <typename Src, int kFilter, int kDepth, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((
-    amdgpu_waves_per_eu(kFilter == kFilterCubic || !IsDenseSource<Src>::value ? 1 : 5)))
+    amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : !IsDenseSource<Src>::value ? 4 : 5)))
 void kRayMarchIntervals(const IteratorContextView *__restrict__ cp,
                                                                   AttrView a, RayMarchIntervalsArgs m)
 {
@@ -72,68 +80,74 @@ void kRayMarchIntervals(const IteratorContextView *__restrict__ cp,
   const F3 d = {m.dir[3 * r], m.dir[3 * r + 1], m.dir[3 * r + 2]};
   IntervalState st;
   intervalInit<kDepth>(c, st, o, d, rayRange(m.tRanges, r));
+  const float dtNominal = st.nominalDeltaT / m.samplingRate;
   float cr = 0.f, cg = 0.f, cb = 0.f, alpha = 0.f;
   uint32_t taken = 0;
-  IntervalOut iv;
-  constexpr int kAhead = samplesAhead<Src>();
-  while (alpha < 0.99f && taken < m.maxSamples && intervalNext<false, kDepth, kQuery>(c, st, iv)) {
-    const float dtNominal = iv.nominalDeltaT / m.samplingRate;
-    float lo = iv.tLower, hi = minf_(iv.tLower + dtNominal, iv.tUpper);
-    if constexpr (kAhead == 1) {
+  auto composite = [&](float s, float dt) {
+    taken++;
+    float rgba[4];
+    tfSampleRgba(m.tf, m.tfSize, m.tfLo, m.tfHi, s, rgba);
+    float op = rgba[3] * dt;
+    op       = op > 0.f ? op : 0.f;
+    op       = op < 1.f ? op : 1.f;
+    cr       = cr + (1.f - alpha) * (rgba[0] * op);
+    cg       = cg + (1.f - alpha) * (rgba[1] * op);
+    cb       = cb + (1.f - alpha) * (rgba[2] * op);
+    alpha    = alpha + (1.f - alpha) * op;
+  };
+  if constexpr (IsDenseSource<Src>::value) {
+    IntervalOut iv;
+    while (alpha < 0.99f && taken < m.maxSamples && intervalNext<false, kDepth, kQuery>(c, st, iv)) {
+      float lo = iv.tLower, hi = minf_(iv.tLower + dtNominal, iv.tUpper);
       while (hi - lo > 0.f && alpha < 0.99f && taken < m.maxSamples) {
-        const float t  = 0.5f * (lo + hi);
-        const float dt = hi - lo;
-        const float s  = smp(F3{o.x + t * d.x, o.y + t * d.y, o.z + t * d.z});
-        taken++;
-        float rgba[4];
-        tfSampleRgba(m.tf, m.tfSize, m.tfLo, m.tfHi, s, rgba);
-        float op = rgba[3] * dt;
-        op       = op > 0.f ? op : 0.f;
-        op       = op < 1.f ? op : 1.f;
-        cr       = cr + (1.f - alpha) * (rgba[0] * op);
-        cg       = cg + (1.f - alpha) * (rgba[1] * op);
-        cb       = cb + (1.f - alpha) * (rgba[2] * op);
-        alpha    = alpha + (1.f - alpha) * op;
-        lo       = hi;
-        hi       = minf_(lo + dtNominal, iv.tUpper);
+        const float t = 0.5f * (lo + hi);
+        composite(smp(F3{o.x + t * d.x, o.y + t * d.y, o.z + t * d.z}), hi - lo);
+        lo = hi;
+        hi = minf_(lo + dtNominal, iv.tUpper);
       }
-    } else {
-      while (hi - lo > 0.f && alpha < 0.99f && taken < m.maxSamples) {
-        // The next kAhead sub-intervals of this interval (the same running
-        // sums as one at a time), their samples issued together so that the
-        // loads overlap, then composited in order with the same stopping
-        // rules; samples past a stop are not counted.
-        float tt[kAhead], dd[kAhead], ss[kAhead];
-        uint32_t nk = 0;
-#pragma unroll
-        for (int k = 0; k < kAhead; k++) {
-          const bool live = hi - lo > 0.f;
-          tt[k]           = 0.5f * (lo + hi);
-          dd[k]           = hi - lo;
-          if (live) {
-            nk = k + 1;
-            lo = hi;
-            hi = minf_(lo + dtNominal, iv.tUpper);
+    }
+  } else {
+    IntervalWalk walk;
+    float lo = 0.f, hi = 0.f, end = 0.f;  // the next sub-interval, the interval's end
+    while (alpha < 0.99f && taken < m.maxSamples) {
+      const uint32_t waiting = (uint32_t)__popcll(__ballot(!(hi - lo > 0.f)));
+      const uint32_t others  = (uint32_t)__popcll(__ballot(hi - lo > 0.f));
+      if (waiting * kMarchIntervalVote >= others) {
+        if (!(hi - lo > 0.f)) {
+          IntervalOut iv;
+          const int event = intervalTick<false, kDepth, kQuery>(c, st, walk, iv);
+          if (event == 2) break;
+          if (event == 1) {
+            lo  = iv.tLower;
+            end = iv.tUpper;
+            hi  = minf_(lo + dtNominal, end);
           }
         }
+      }
+      if (!(hi - lo > 0.f)) continue;
+      // The next kSamplesAhead sub-intervals (the same running sums as one
+      // at a time), their samples issued together so that the loads overlap,
+      // then composited in order with the same stopping rules; samples past
+      // a stop are not counted.
+      float tt[kSamplesAhead], dd[kSamplesAhead], ss[kSamplesAhead];
+      uint32_t nk = 0;
 #pragma unroll
-        for (int k = 0; k < kAhead; k++)
-          ss[k] = (uint32_t)k < nk ? smp(F3{o.x + tt[k] * d.x, o.y + tt[k] * d.y, o.z + tt[k] * d.z}) : 0.f;
-#pragma unroll
-        for (int k = 0; k < kAhead; k++) {
-          if ((uint32_t)k >= nk || !(alpha < 0.99f) || taken >= m.maxSamples) continue;
-          taken++;
-          float rgba[4];
-          tfSampleRgba(m.tf, m.tfSize, m.tfLo, m.tfHi, ss[k], rgba);
-          float op = rgba[3] * dd[k];
-          op       = op > 0.f ? op : 0.f;
-          op       = op < 1.f ? op : 1.f;
-          cr       = cr + (1.f - alpha) * (rgba[0] * op);
-          cg       = cg + (1.f - alpha) * (rgba[1] * op);
-          cb       = cb + (1.f - alpha) * (rgba[2] * op);
-          alpha    = alpha + (1.f - alpha) * op;
+      for (int k = 0; k < kSamplesAhead; k++) {
+        const bool live = hi - lo > 0.f;
+        tt[k]           = 0.5f * (lo + hi);
+        dd[k]           = hi - lo;
+        if (live) {
+          nk = k + 1;
+          lo = hi;
+          hi = minf_(lo + dtNominal, end);
         }
       }
+#pragma unroll
+      for (int k = 0; k < kSamplesAhead; k++)
+        ss[k] = (uint32_t)k < nk ? smp(F3{o.x + tt[k] * d.x, o.y + tt[k] * d.y, o.z + tt[k] * d.z}) : 0.f;
+#pragma unroll
+      for (int k = 0; k < kSamplesAhead; k++)
+        if ((uint32_t)k < nk && alpha < 0.99f && taken < m.maxSamples) composite(ss[k], dd[k]);
     }
   }
   m.rgba[4 * r]     = cr;
@@ -144,7 +158,9 @@ void kRayMarchIntervals(const IteratorContextView *__restrict__ cp,
 }
 
 // Launches the instantiation for the context's iterator depth on vdb
-// sources (the DDA keeps only the levels it walks) and for its query kind
+// sources (the DDA keeps only the levels it walks; on structuredRegular ones
+// for the default depth, whose DDA step then needs no re-initialisation: 5.1
+// -> 4.9 ms a 1080p frame of the 512^3 volume) and for its query kind
 // (denseQueryOf: structuredRegular volumes within one level-1 node use the
 // dense node numbering, and their kernels then carry no node-table query).
 struct RayMarchIntervalsLaunch
@@ -165,9 +181,8 @@ struct RayMarchIntervalsLaunch
   template <typename Src, int kFilter>
   hipError_t operator()() const
   {
-    // structuredRegular sources keep the depth-generic kernel, which
-    // measured faster for them (5.1 against 5.6 ms per 1080p frame).
     if constexpr (IsDenseSource<Src>::value) {
+      if (denseQuery && depth == 2) return run<Src, kFilter, 2, 1>();
       return denseQuery ? run<Src, kFilter, -1, 1>() : run<Src, kFilter, -1, 0>();
     } else {
       switch (depth) {

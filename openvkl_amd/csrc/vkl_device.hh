@@ -900,6 +900,45 @@ VKL_DEV F3 gradientCubic(const Src &src, F3 p)
   return cubicGradientFromTaps(S, p, ic);
 }
 
+// gradientCubic with one x slice of the stencil (16 taps) alive at a time:
+// the same sums in the same order. For kernels that keep much state of their
+// own across the call, where 64 live taps would push that state to scratch.
+template <typename Src>
+VKL_DEV F3 gradientCubicBySlices(const Src &src, F3 p)
+{
+  const I3 ic = {floorToInt(p.x), floorToInt(p.y), floorToInt(p.z)};
+  const F3 d  = {p.x - (float)ic.x, p.y - (float)ic.y, p.z - (float)ic.z};
+  float wx[4], wy[4], wz[4], dx[4], dy[4], dz[4];
+  crWeights(d.x, wx);
+  crWeights(d.y, wy);
+  crWeights(d.z, wz);
+  crDerivWeights(d.x, dx);
+  crDerivWeights(d.y, dy);
+  crDerivWeights(d.z, dz);
+  F3 g = {0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int i = 0; i < 4; i++) {
+    const float wi = i == 0 ? wx[0] : i == 1 ? wx[1] : i == 2 ? wx[2] : wx[3];
+    const float di = i == 0 ? dx[0] : i == 1 ? dx[1] : i == 2 ? dx[2] : dx[3];
+    float gy_v = 0.f, gy_dy = 0.f, gy_dz = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      float q[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) q[k] = src.at(ic.x + i - 1, ic.y + j - 1, ic.z + k - 1);
+      const float vz  = wz[0] * q[0] + wz[1] * q[1] + wz[2] * q[2] + wz[3] * q[3];
+      const float dzv = dz[0] * q[0] + dz[1] * q[1] + dz[2] * q[2] + dz[3] * q[3];
+      gy_v += wy[j] * vz;
+      gy_dy += dy[j] * vz;
+      gy_dz += wy[j] * dzv;
+    }
+    g.x += di * gy_v;
+    g.y += wi * gy_dy;
+    g.z += wi * gy_dz;
+  }
+  return g;
+}
+
 // Tricubic in the stream kernels (kSample, kGradient): vdb sources gather
 // their taps by leaf cells (cubicTapsByLeafCells). The fused ray and
 // iterator kernels keep the per-tap reads of sampleCubic: inlined at their
@@ -1016,6 +1055,10 @@ VKL_DEV int32_t clampCell(float f, int32_t res) { return floorToInt(vmax(f, 0.f)
 
 constexpr uint32_t kMaxDdaSteps = 1u << 22;
 
+// Lanes of a wavefront that wait for the interval phase of hitTick, times
+// this, against the lanes that have a sample to take.
+constexpr uint32_t kHitIntervalVote = 3;
+
 #define DX(l) (l)
 #define DY(l) (4 + (l))
 #define DZ(l) (8 + (l))
@@ -1074,37 +1117,16 @@ VKL_DEV void ddaInit(DdaState &d, F3 org, F3 dir, float tMin, uint32_t level)
   }
 }
 
-// Dda.ih:204-266: levels L + 1 .. d.level restart from the current t, nudged
-// 1e-2 across the plane the level-L step crossed.
-template <int kDepth, int L>
-VKL_DEV void ddaReinitBelow(DdaState &d, int32_t dx, int32_t dy)
+// Signed 1 / dir of an axis as dirRcp gives it, from its stored magnitude.
+VKL_DEV float ddaRcp(const DdaState &d, int axis)
 {
-  const F3 dir = {d.rayDir[0], d.rayDir[1], d.rayDir[2]};
-  const F3 id  = {dirRcp(dir.x), dirRcp(dir.y), dirRcp(dir.z)};
-  const int sx = dirSign(dir.x), sy = dirSign(dir.y), sz = dirSign(dir.z);
-  F3 oo = {d.rayOrg[0] + d.t * dir.x, d.rayOrg[1] + d.t * dir.y, d.rayOrg[2] + d.t * dir.z};
-  if (dx != 0)
-    oo.x = oo.x + ((float)sx) * 1e-2f;
-  else if (dy != 0)
-    oo.y = oo.y + ((float)sy) * 1e-2f;
-  else
-    oo.z = oo.z + ((float)sz) * 1e-2f;
-#pragma unroll
-  for (int l = L + 1; l < 4; ++l) {
-    if ((uint32_t)l > ddaLevel<kDepth>(d)) continue;
-    const int32_t res = (int32_t)kRes[l + 1];
-    d.idx[DX(l)]      = clampCell(oo.x, res);
-    d.idx[DY(l)]      = clampCell(oo.y, res);
-    d.idx[DZ(l)]      = clampCell(oo.z, res);
-    d.tNext[DX(l)]    = planeT((float)(d.idx[DX(l)] + res * (sx >= 0)), d.rayOrg[0], id.x);
-    d.tNext[DY(l)]    = planeT((float)(d.idx[DY(l)] + res * (sy >= 0)), d.rayOrg[1], id.y);
-    d.tNext[DZ(l)]    = planeT((float)(d.idx[DZ(l)] + res * (sz >= 0)), d.rayOrg[2], id.z);
-  }
+  return d.rayDir[axis] < 0.f ? -d.absRcp[axis] : d.absRcp[axis];
 }
 
-// Dda.ih:271-309 (ties: x, then y, then z).
+// Dda.ih:271-309 (ties: x, then y, then z). Returns the axis along which the
+// cell moved (z when it did not).
 template <int L>
-VKL_DEV void ddaStep(DdaState &d)
+VKL_DEV int ddaStep(DdaState &d)
 {
   // Every field is written on every path (values selected, not addresses),
   // so the state stays in registers.
@@ -1118,56 +1140,80 @@ VKL_DEV void ddaStep(DdaState &d)
   d.tNext[DX(L)]    = sx ? tx + ddaTDelta<L>(d, 0) : tx;
   d.tNext[DY(L)]    = sy ? ty + ddaTDelta<L>(d, 1) : ty;
   d.tNext[DZ(L)]    = sz ? tz + ddaTDelta<L>(d, 2) : tz;
-  d.idx[DX(L)]      = d.idx[DX(L)] + (sx ? dirSign(d.rayDir[0]) * res : 0);
-  d.idx[DY(L)]      = d.idx[DY(L)] + (sy ? dirSign(d.rayDir[1]) * res : 0);
+  const int32_t mx  = sx ? dirSign(d.rayDir[0]) * res : 0;
+  const int32_t my  = sy ? dirSign(d.rayDir[1]) * res : 0;
+  d.idx[DX(L)]      = d.idx[DX(L)] + mx;
+  d.idx[DY(L)]      = d.idx[DY(L)] + my;
   d.idx[DZ(L)]      = d.idx[DZ(L)] + (sz ? dirSign(d.rayDir[2]) * res : 0);
+  return mx ? 0 : (my ? 1 : 2);
 }
 
-// HDDA.ih.in:52-101, parents of a stepped level from the nearest one up:
+// Level l restarts at the position oo (Dda.ih:235-260).
+template <int l>
+VKL_DEV void ddaReinitLevel(DdaState &d, F3 oo)
+{
+  const int32_t res = (int32_t)kRes[l + 1];
+  d.idx[DX(l)]      = clampCell(oo.x, res);
+  d.idx[DY(l)]      = clampCell(oo.y, res);
+  d.idx[DZ(l)]      = clampCell(oo.z, res);
+  d.tNext[DX(l)]    = planeT((float)(d.idx[DX(l)] + (d.rayDir[0] < 0.f ? 0 : res)), d.rayOrg[0], ddaRcp(d, 0));
+  d.tNext[DY(l)]    = planeT((float)(d.idx[DY(l)] + (d.rayDir[1] < 0.f ? 0 : res)), d.rayOrg[1], ddaRcp(d, 1));
+  d.tNext[DZ(l)]    = planeT((float)(d.idx[DZ(l)] + (d.rayDir[2] < 0.f ? 0 : res)), d.rayOrg[2], ddaRcp(d, 2));
+}
+
+// HDDA.ih.in:52-101, parents of the stepped level L from the nearest one up:
 // each one steps only if its child left its cell.
 template <int P>
-VKL_DEV void hddaParents(DdaState &d)
+VKL_DEV void hddaParents(DdaState &d, uint32_t L)
 {
   if constexpr (P >= 0) {
-    constexpr int C   = P + 1;
-    const int32_t res = (int32_t)kRes[P + 1];
-    const bool left   = d.idx[DX(C)] < d.idx[DX(P)] || d.idx[DY(C)] < d.idx[DY(P)] || d.idx[DZ(C)] < d.idx[DZ(P)] ||
-                      d.idx[DX(C)] >= d.idx[DX(P)] + res || d.idx[DY(C)] >= d.idx[DY(P)] + res ||
-                      d.idx[DZ(C)] >= d.idx[DZ(P)] + res;
-    if (!left) return;
-    ddaStep<P>(d);
-    hddaParents<P - 1>(d);
+    bool follow = true;
+    if ((uint32_t)P < L) {
+      constexpr int C   = P + 1;
+      const int32_t res = (int32_t)kRes[P + 1];
+      follow = d.idx[DX(C)] < d.idx[DX(P)] || d.idx[DY(C)] < d.idx[DY(P)] || d.idx[DZ(C)] < d.idx[DZ(P)] ||
+               d.idx[DX(C)] >= d.idx[DX(P)] + res || d.idx[DY(C)] >= d.idx[DY(P)] + res ||
+               d.idx[DZ(C)] >= d.idx[DZ(P)] + res;
+      if (follow) (void)ddaStep<P>(d);
+    }
+    if (follow) hddaParents<P - 1>(d, L);
   }
 }
 
-// HDDA.ih.in:24-101: step on level L (the level of the empty voxel),
-// re-initialise the levels below, and let parents follow a child that left
-// their cell.
-template <int kDepth, int L>
-VKL_DEV void hddaStepAt(DdaState &d)
-{
-  if constexpr (L >= 3) {
-    ddaStep<3>(d);
-  } else {
-    const int32_t ox = d.idx[DX(L)], oy = d.idx[DY(L)];
-    ddaStep<L>(d);
-    if ((uint32_t)L < ddaLevel<kDepth>(d)) ddaReinitBelow<kDepth, L>(d, d.idx[DX(L)] - ox, d.idx[DY(L)] - oy);
-  }
-  hddaParents<(L >= 3 ? 3 : L) - 1>(d);
-}
-
-// descLevel never exceeds the DDA's deepest level (queries descend no
-// deeper), so with a compile-time depth the deeper cases are not generated.
+// HDDA.ih.in:24-101: step on level L (the level of the empty voxel, never
+// deeper than the DDA's deepest), re-initialise the levels below from the
+// current t nudged 1e-2 across the plane the step crossed (Dda.ih:204-266),
+// and let parents follow a child that left their cell. Only the step itself
+// is a switch over the level; the re-initialisation of a level and the
+// parents' steps each have one body that lanes stepping on different levels
+// share, because the lanes of a wavefront rarely step on the same level (with
+// a body per level, 3 to 9 of 64 lanes were active).
 template <int kDepth>
-VKL_DEV void hddaStep(DdaState &d, uint32_t descLevel)
+VKL_DEV void hddaStep(DdaState &d, uint32_t L)
 {
   constexpr int kMax = kDepth >= 0 ? kDepth : 3;
-  switch (descLevel) {
-  case 0: hddaStepAt<kDepth, 0>(d); break;
-  case 1: hddaStepAt<kDepth, (kMax < 1 ? kMax : 1)>(d); break;
-  case 2: hddaStepAt<kDepth, (kMax < 2 ? kMax : 2)>(d); break;
-  default: hddaStepAt<kDepth, kMax>(d); break;
+  int axis;
+  if (L == 0)
+    axis = ddaStep<0>(d);
+  else if (kMax >= 2 && L == 1)
+    axis = ddaStep<(kMax < 1 ? kMax : 1)>(d);
+  else if (kMax >= 3 && L == 2)
+    axis = ddaStep<(kMax < 2 ? kMax : 2)>(d);
+  else
+    axis = ddaStep<kMax>(d);
+  if (L < ddaLevel<kDepth>(d)) {
+    F3 oo = {d.rayOrg[0] + d.t * d.rayDir[0], d.rayOrg[1] + d.t * d.rayDir[1], d.rayOrg[2] + d.t * d.rayDir[2]};
+    if (axis == 0)
+      oo.x = oo.x + (float)dirSign(d.rayDir[0]) * 1e-2f;
+    else if (axis == 1)
+      oo.y = oo.y + (float)dirSign(d.rayDir[1]) * 1e-2f;
+    else
+      oo.z = oo.z + (float)dirSign(d.rayDir[2]) * 1e-2f;
+    if (kMax >= 1 && L < 1 && 1 <= ddaLevel<kDepth>(d)) ddaReinitLevel<1>(d, oo);
+    if (kMax >= 2 && L < 2 && 2 <= ddaLevel<kDepth>(d)) ddaReinitLevel<2>(d, oo);
+    if (kMax >= 3 && L < 3 && 3 <= ddaLevel<kDepth>(d)) ddaReinitLevel<3>(d, oo);
   }
+  hddaParents<kMax - 1>(d, L);
 }
 
 // Pins a value to a register: the optimizer can no longer turn a select
@@ -1327,41 +1373,69 @@ VKL_DEV bool denseQuery(const GridView &g)
   return g.dense != 0 && g.activeSize[0] <= kRes[1] && g.activeSize[1] <= kRes[1] && g.activeSize[2] <= kRes[1];
 }
 
-// VdbIterator_iterateIntervalInternal, VdbIterator.ispc:96-159. kQuery: 0
-// the general query, 1 the dense one, -1 chosen per context at run time.
-template <bool kNodeCache = false, int kDepth = -1, int kQuery = -1>
-VKL_DEV bool intervalNext(const IteratorContextView &c, IntervalState &it, IntervalOut &out)
+// What an interval walk keeps beside the state of the caller.
+struct IntervalWalk
 {
-  if (!(it.dda.t <= it.tMax)) return false;
-  const bool dense = kQuery >= 0 ? kQuery == 1 : denseQuery(c.sampler.grid);
-  VoxelDesc v{0, true, {0.f, 0.f}};
-  // Every step advances t by a positive tDelta; a ray whose step makes no
+  uint32_t steps;    // voxels visited since the last interval
+  bool inLeaf;       // depth 3: the next cell lies in the leaf of the last query,
+  Range1f leafRange;  // whose value range this is
+
+  VKL_DEV IntervalWalk() : steps(0), inLeaf(false), leafRange{0.f, 0.f} {}
+};
+
+// One voxel of VdbIterator_iterateIntervalInternal (VdbIterator.ispc:96-159):
+// 0 the voxel was empty, 1 `out` holds its interval, 2 the ray has ended.
+// The lanes of a wavefront take one voxel each per call, and there is one
+// query and one DDA step for empty and occupied voxels alike, so lanes with
+// an interval do not wait for the ones still crossing empty space. kQuery: 0
+// the general query, 1 the dense one, -1 chosen per context at run time.
+template <bool kNodeCache, int kDepth, int kQuery>
+VKL_DEV int intervalTick(const IteratorContextView &c, IntervalState &it, IntervalWalk &w, IntervalOut &out)
+{
+  DdaState &dda = it.dda;
+  // Every step advances t by a positive tDelta; a ray whose steps make no
   // progress (infinite direction components) is ended after kMaxDdaSteps.
-  uint32_t steps = 0;
-  while (it.dda.t <= it.tMax) {
-    if (++steps > kMaxDdaSteps) {
-      it.tMax = -vinf();
-      return false;
-    }
-    const uint32_t l = ddaLevel<kDepth>(it.dda);
-    const I3 cell    = ddaCell<kDepth>(it.dda);
-    if (dense)
+  if (!(dda.t <= it.tMax) || ++w.steps > kMaxDdaSteps) return 2;
+  const I3 cell = ddaCell<kDepth>(dda);
+  VoxelDesc v{3u, false, w.leafRange};
+  if (kDepth != 3 || !w.inLeaf) {
+    const uint32_t l = ddaLevel<kDepth>(dda);
+    if (kQuery >= 0 ? kQuery == 1 : denseQuery(c.sampler.grid))
       queryVoxelDense(c, cell.x, cell.y, cell.z, l, v);
     else
       queryVoxel<kNodeCache>(c, cell.x, cell.y, cell.z, l, v, it);
-    if (!v.isEmpty) break;
-    hddaStep<kDepth>(it.dda, v.level);
   }
-  if (it.dda.t < it.tMax) {
-    out.vLower = v.valueRange.lower;
-    out.vUpper = v.valueRange.upper;
-    out.tLower = it.dda.t;
-    hddaStep<kDepth>(it.dda, v.level);
-    out.tUpper        = vmin(it.dda.t, it.tMax);
-    out.nominalDeltaT = it.nominalDeltaT;
-    return true;
+  const float tLower = dda.t;
+  hddaStep<kDepth>(dda, v.level);
+  if (kDepth == 3) {
+    // The voxels of a leaf share one query result (its majorant).
+    const I3 to = ddaCell<kDepth>(dda);
+    w.inLeaf    = !v.isEmpty && v.level == 3u &&
+               (uint32_t)((cell.x ^ to.x) | (cell.y ^ to.y) | (cell.z ^ to.z)) < kRes[3];
+    w.leafRange = v.valueRange;
   }
-  return false;
+  if (v.isEmpty) return 0;
+  if (!(tLower < it.tMax)) return 2;
+  w.steps           = 0;
+  out.vLower        = v.valueRange.lower;
+  out.vUpper        = v.valueRange.upper;
+  out.tLower        = tLower;
+  out.tUpper        = vmin(dda.t, it.tMax);
+  out.nominalDeltaT = it.nominalDeltaT;
+  return 1;
+}
+
+// The next interval of one ray.
+template <bool kNodeCache = false, int kDepth = -1, int kQuery = -1>
+VKL_DEV bool intervalNext(const IteratorContextView &c, IntervalState &it, IntervalOut &out)
+{
+  IntervalWalk w;
+  int event;
+  do
+    event = intervalTick<kNodeCache, kDepth, kQuery>(c, it, w, out);
+  while (event == 0);
+  if (event == 2) it.tMax = -vinf();
+  return event == 1;
 }
 
 // ---- hit iteration (DefaultIterator.ispc:141-258, Iterator.ih:17-200) --------
@@ -1370,89 +1444,6 @@ template <typename S>
 VKL_DEV float sampleAlong(const S &smp, F3 o, F3 d, float t)
 {
   return smp(F3{o.x + t * d.x, o.y + t * d.y, o.z + t * d.z});
-}
-
-// bisect, Iterator.ih:23-85.
-template <typename S>
-VKL_DEV float bisect(const S &smp, F3 o, F3 d, float t0, float s0, float t, float s, float iso, float tol)
-{
-  float tMid = 0.f;
-#pragma unroll 1
-  for (int iter = 0; iter < 10; ++iter) {
-    tMid            = 0.5f * (t0 + t);
-    const float err = 0.5f * (t - t0);
-    if (err < tol) break;
-    const float sm = sampleAlong(smp, o, d, tMid);
-    if (isnan(sm)) return (fabsf(iso - s0) < fabsf(iso - s)) ? t0 : t;
-    if (sm == iso || (iso - s0) * (iso - sm) < 0.f) {
-      t = tMid;
-      s = sm;
-    } else if (s == iso || (iso - s) * (iso - sm) < 0.f) {
-      t0 = tMid;
-      s0 = sm;
-    } else {
-      return vinf();
-    }
-  }
-  return tMid;
-}
-
-// intersectSurfacesBisection, Iterator.ih:87-197.
-template <typename S>
-VKL_DEV bool intersectBisection(const IteratorContextView &c, const S &smp, F3 o, F3 d, float tLo, float tHi,
-                                float step, HitOut &hit)
-{
-  float t0 = tLo;
-  float s0 = sampleAlong(smp, o, d, t0);
-  for (int it = 0; it < 10 && isnan(s0) && t0 < tHi; ++it) {
-    t0 += vmax(1e-5f, 1e-5f * step);
-    s0 = sampleAlong(smp, o, d, t0);
-  }
-  while (t0 < tHi) {
-    const float h = vmin(step, tHi - t0);
-    const float t = t0 + h;
-    if (!(t > t0)) break;  // no float progress: the march cannot continue
-    float s       = sampleAlong(smp, o, d, t);
-    float ts      = t;
-    for (int it = 0; it < 10 && isnan(s) && ts > t0; ++it) {
-      ts -= vmax(1e-5f, 1e-5f * step);
-      s = sampleAlong(smp, o, d, ts);
-    }
-    float tHit = vinf(), eps = vinf(), value = vinf();
-    for (int i = 0; i < c.numValues; i++) {
-      const float v = c.values[i];
-      if (fabsf(s0 - v) < 1e-6f) {
-        if (t0 < tHit && t0 <= tHi) {
-          tHit  = t0;
-          value = v;
-          eps   = 0.125f * step;
-        }
-      } else if (!isnan(s0 + s) && (v - s0) * (v - s) < 0.f) {
-        const float tIso = bisect(smp, o, d, t0, s0, ts, s, v, vmin(1e-6f, 0.01f * h));
-        if (tIso < tHit && tIso <= tHi) {
-          tHit  = tIso;
-          value = v;
-          eps   = 0.125f * step;
-        }
-      }
-      if (t == tHi && fabsf(s - v) < 1e-6f) {
-        if (ts < tHit && ts <= tHi) {
-          tHit  = ts;
-          value = v;
-          eps   = 0.125f * step;
-        }
-      }
-    }
-    if (tHit < vinf()) {
-      hit.t       = tHit;
-      hit.sample  = value;
-      hit.epsilon = eps * sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
-      return true;
-    }
-    t0 = t;
-    s0 = s;
-  }
-  return false;
 }
 
 template <int kDepth = -1>
@@ -1472,42 +1463,272 @@ VKL_DEV void hitInit(const IteratorContextView &c, HitState &h, F3 origin, F3 di
   h.lastHitOffsetT   = -vinf();
 }
 
-// DefaultHitIterator_iterateHit, DefaultIterator.ispc:168-258.
+// A ray's hit iteration as a state machine that advances one voxel query or
+// one sample at a time (hitTick). The lanes of a wavefront are in different
+// phases of the reference's nested loops (intervals, the march through one,
+// bisection) most of the time; run as nested loops, every lane waits for the
+// longest inner loop of its wavefront (3.3 of 64 lanes active on a 1024^3
+// vdb, 8.7 in the hit renderer). Here every lane advances at each tick, all
+// samples (start, march, bisection) share one sampler call, and the kernels
+// hold one copy of the query, the DDA step and the sampler.
+struct HitSearch
+{
+  HitState h;
+  uint32_t mode;      // what the ray waits for
+  uint32_t tries;     // NaN retries or bisection probes done
+  IntervalWalk walk;
+  float tp;           // position of the pending sample
+  float t0, s0;       // start of the march step and its sample
+  float tKnown;       // position s0 was taken at
+  float t;            // end of the march step
+  // What only a bisection keeps from tick to tick, one LDS word each at
+  // bisect[word * kHitLanes] (in registers these 10 words cost the kernels an
+  // occupancy step or as much scratch).
+  float *bisect;
+};
+
+constexpr uint32_t kHitLanes = 64;  // lanes of a block that searches
+enum : uint32_t
+{
+  kBisT0    = 0,  // the bracket and its samples
+  kBisS0    = 1,
+  kBisT1    = 2,
+  kBisS1    = 3,
+  kBisTol   = 4,
+  kBisTs    = 5,  // position and value of the march sample
+  kBisS     = 6,
+  kBisHit   = 7,  // nearest hit of the step so far and its iso value
+  kBisValue = 8,
+  kBisIso   = 9,  // index of the iso value being bisected
+  kBisWords = 10
+};
+
+enum : uint32_t
+{
+  kHitInterval = 0,  // the next interval
+  kHitStart    = 1,  // the sample at the start of a range
+  kHitMarch    = 2,  // the sample at the end of a march step
+  kHitBisect   = 3,  // a bisection probe
+  kHitDone     = 4,
+};
+
+// Start or resume the search of h (DefaultIterator.ispc:186-200).
+VKL_DEV void hitResume(HitSearch &q)
+{
+  q.tries = 0;
+  q.t0 = q.tp = q.h.curLower;
+  q.mode      = q.h.curLower == vinf() ? kHitDone : (q.h.curUpper <= q.h.curLower ? kHitInterval : kHitStart);
+}
+
+// `bisect`: the lane's first word of kBisWords * kHitLanes floats of LDS.
+VKL_DEV void hitBegin(HitSearch &q, float *bisect)
+{
+  q.walk   = IntervalWalk();
+  q.bisect = bisect;
+  q.tKnown = __builtin_nanf("");
+  q.s0     = 0.f;
+  hitResume(q);
+}
+
+// The next march step from (t0, s0), Iterator.ih:113-125; past the range's
+// end, or without float progress, the next interval.
+VKL_DEV void hitMarch(HitSearch &q)
+{
+  q.t     = q.t0 + vmin(q.h.iv.nominalDeltaT, q.h.curUpper - q.t0);
+  q.tp    = q.t;
+  q.tries = 0;
+  q.mode  = kHitMarch;
+  if (!(q.t0 < q.h.curUpper && q.t > q.t0)) {
+    q.h.curLower = vinf();
+    q.mode       = kHitInterval;
+  }
+}
+
+// One tick; every lane of the wavefront that still searches calls it
+// together. 0: still searching, 1: `hit` holds the next hit, 2: no more hits.
+template <typename S, int kQuery = -1>
+VKL_DEV int hitTick(const IteratorContextView &c, const S &smp, HitSearch &q, HitOut &hit)
+{
+  constexpr int kDepth = hitDepthOf<typename S::Source>();
+  HitState &h          = q.h;
+  int event            = 0;
+  if (q.mode == kHitDone || c.numValues == 0) return 2;
+
+  // The interval phase runs for a wavefront once a quarter of its searching
+  // lanes wait for it (or none has a sample to take): running it for one or
+  // two lanes costs as many instructions as for all.
+  const uint32_t waiting = (uint32_t)__popcll(__ballot(q.mode == kHitInterval));
+  const uint32_t others  = (uint32_t)__popcll(__ballot(q.mode != kHitInterval));
+  if (waiting * kHitIntervalVote >= others) {
+    if (q.mode == kHitInterval) {
+      IntervalOut iv;
+      const int found = intervalTick<true, kDepth, kQuery>(c, h.iv, q.walk, iv);
+      if (found == 2) event = 2;
+      if (found == 1) {
+        h.curLower         = vmax(iv.tLower, h.lastHitOffsetT);
+        h.curUpper         = iv.tUpper;
+        h.curNominalDeltaT = iv.nominalDeltaT;  // the caller's state; the search reads iv's
+        if (!(h.curUpper <= h.curLower)) {
+          // Adjoining ranges share their end sample.
+          q.t0    = h.curLower;
+          q.tp    = h.curLower;
+          q.tries = 0;
+          q.mode  = kHitStart;
+          if (q.t0 == q.tKnown && !isnan(q.s0)) hitMarch(q);
+        }
+      }
+    }
+  }
+
+  // The sample phase: the sample each lane waits for, and what follows
+  // from it (bisect and intersectSurfacesBisection, Iterator.ih:23-197).
+  if (event == 0 && q.mode != kHitInterval) {
+    const F3 o      = {h.origin[0], h.origin[1], h.origin[2]};
+    const F3 d      = {h.direction[0], h.direction[1], h.direction[2]};
+    const float sm  = sampleAlong(smp, o, d, q.tp);
+    const float tHi = h.curUpper, step = h.iv.nominalDeltaT;
+    float *bis      = q.bisect;
+    bool compare = false, resumed = false, go = false;
+    // The march sample under comparison, the nearest hit so far.
+    float ts = q.tp, s = sm, tHit = vinf(), value = vinf();
+    int iso = 0;
+    if (q.mode == kHitBisect) {
+      float b0 = bis[kBisT0 * kHitLanes], c0 = bis[kBisS0 * kHitLanes];
+      float b1 = bis[kBisT1 * kHitLanes], c1 = bis[kBisS1 * kHitLanes];
+      iso         = __float_as_int(bis[kBisIso * kHitLanes]);
+      const float v = c.values[iso];
+      float tIso    = vinf();
+      bool more     = false;
+      if (isnan(sm)) {
+        tIso = (fabsf(v - c0) < fabsf(v - c1)) ? b0 : b1;
+      } else if (sm == v || (v - c0) * (v - sm) < 0.f) {
+        b1   = q.tp;
+        c1   = sm;
+        more = true;
+      } else if (c1 == v || (v - c1) * (v - sm) < 0.f) {
+        b0   = q.tp;
+        c0   = sm;
+        more = true;
+      }
+      if (more) {
+        tIso = q.tp;
+        more = ++q.tries < 10u;
+        if (more) {
+          q.tp = 0.5f * (b0 + b1);
+          if (0.5f * (b1 - b0) < bis[kBisTol * kHitLanes]) {
+            tIso = q.tp;
+            more = false;
+          }
+        }
+      }
+      if (more) {
+        bis[kBisT0 * kHitLanes] = b0;
+        bis[kBisS0 * kHitLanes] = c0;
+        bis[kBisT1 * kHitLanes] = b1;
+        bis[kBisS1 * kHitLanes] = c1;
+      } else {
+        ts    = bis[kBisTs * kHitLanes];
+        s     = bis[kBisS * kHitLanes];
+        tHit  = bis[kBisHit * kHitLanes];
+        value = bis[kBisValue * kHitLanes];
+        if (tIso < tHit && tIso <= tHi) {
+          tHit  = tIso;
+          value = v;
+        }
+        compare = resumed = true;
+      }
+    } else if (isnan(sm) && q.tries < 10u && (q.mode == kHitStart ? q.t0 < tHi : ts > q.t0)) {
+      const float nudge = vmax(1e-5f, 1e-5f * step);
+      q.tries++;
+      q.tp = q.mode == kHitStart ? q.t0 + nudge : ts - nudge;
+      if (q.mode == kHitStart) q.t0 = q.tp;
+    } else if (q.mode == kHitStart) {
+      q.s0     = sm;
+      q.tKnown = q.t0;
+      go       = true;
+    } else {
+      compare = true;
+    }
+    if (compare) {
+      for (int i = 0; i < c.numValues; i++) {
+        const float v = c.values[i];
+        if (!compare || i < iso) continue;
+        if (!(resumed && i == iso)) {
+          if (fabsf(q.s0 - v) < 1e-6f) {
+            if (q.t0 < tHit && q.t0 <= tHi) {
+              tHit  = q.t0;
+              value = v;
+            }
+          } else if (!isnan(q.s0 + s) && (v - q.s0) * (v - s) < 0.f) {
+            const float tol = vmin(1e-6f, 0.01f * vmin(step, tHi - q.t0));
+            q.tp            = 0.5f * (q.t0 + ts);
+            if (0.5f * (ts - q.t0) < tol) {
+              if (q.tp < tHit && q.tp <= tHi) {
+                tHit  = q.tp;
+                value = v;
+              }
+            } else {
+              bis[kBisT0 * kHitLanes]    = q.t0;
+              bis[kBisS0 * kHitLanes]    = q.s0;
+              bis[kBisT1 * kHitLanes]    = ts;
+              bis[kBisS1 * kHitLanes]    = s;
+              bis[kBisTol * kHitLanes]   = tol;
+              bis[kBisTs * kHitLanes]    = ts;
+              bis[kBisS * kHitLanes]     = s;
+              bis[kBisHit * kHitLanes]   = tHit;
+              bis[kBisValue * kHitLanes] = value;
+              bis[kBisIso * kHitLanes]   = __int_as_float(i);
+              q.tries = 0;
+              q.mode  = kHitBisect;
+              compare = false;
+              continue;
+            }
+          }
+        }
+        if (q.t == tHi && fabsf(s - v) < 1e-6f) {
+          if (ts < tHit && ts <= tHi) {
+            tHit  = ts;
+            value = v;
+          }
+        }
+      }
+    }
+    if (compare) {
+      if (tHit < vinf()) {
+        hit.t            = tHit;
+        hit.sample       = value;
+        hit.epsilon      = 0.125f * step * sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
+        h.curLower       = hit.t + hit.epsilon;
+        h.lastHitOffsetT = hit.t + hit.epsilon;
+        hitResume(q);
+        event = 1;
+      } else {
+        q.t0     = q.t;
+        q.s0     = s;
+        q.tKnown = ts;
+        go       = true;
+      }
+    }
+    if (go) hitMarch(q);
+  }
+  return event;
+}
+
+// DefaultHitIterator_iterateHit, DefaultIterator.ispc:168-258, for one ray.
 template <typename S, int kQuery = -1>
 VKL_DEV bool hitNext(const IteratorContextView &c, const S &smp, HitState &h, HitOut &hit)
 {
-  if (c.numValues == 0) return false;
-  if (h.curLower == vinf()) return false;
-  const F3 o = {h.origin[0], h.origin[1], h.origin[2]};
-  const F3 d = {h.direction[0], h.direction[1], h.direction[2]};
-  for (;;) {
-    const bool need = h.curUpper <= h.curLower;
-    bool have       = !need;
-    if (need) {
-      IntervalOut iv;
-      have = intervalNext<true, hitDepthOf<typename S::Source>(), kQuery>(c, h.iv, iv);
-      if (have) {
-        h.curLower         = iv.tLower;
-        h.curUpper         = iv.tUpper;
-        h.curNominalDeltaT = iv.nominalDeltaT;
-      }
-    }
-    if (need && have) {
-      h.curLower = vmax(h.curLower, h.lastHitOffsetT);
-      if (h.curUpper <= h.curLower) continue;
-    }
-    if (!have) {
-      h.curLower = vinf();
-      return false;
-    }
-    hit.t = vinf();
-    if (intersectBisection(c, smp, o, d, h.curLower, h.curUpper, h.curNominalDeltaT, hit)) {
-      h.curLower       = hit.t + hit.epsilon;
-      h.lastHitOffsetT = hit.t + hit.epsilon;
-      return true;
-    }
-    h.curLower = vinf();
-  }
+  __shared__ float bisect[kBisWords * kHitLanes];
+  HitSearch q;
+  q.h = h;
+  hitBegin(q, bisect);
+  int event;
+  do
+    event = hitTick<S, kQuery>(c, smp, q, hit);
+  while (event == 0);
+  if (event == 2) q.h.curLower = vinf();
+  h = q.h;
+  return event == 1;
 }
 
 }  // namespace vklhip

@@ -1,0 +1,81 @@
+"""Interval and hit iteration where a lane's walk takes its rarer turns: rays
+along an axis (zero direction components of both signs) and on cell planes,
+leaves beside tiles on every level, undefined voxels inside a march (the NaN
+retries), several iso values in one step, plateaus at an iso value, ranges that
+end inside a cell, batches of one ray and of a wavefront and one. Bit-identical
+to the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+from tests import volumes as V
+from tests.test_gpu_iterators import compare_intervals, rays_through
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def dense_pair(device):
+    rng = np.random.default_rng(21)
+    data = V.procedural((45, 38, 51), lambda x, y, z: np.sin(0.4 * x) * np.cos(0.3 * y) + 0.02 * z)
+    data[rng.random(data.shape) < 0.002] = np.nan
+    data[10:20, 10:20, 10:20] = 0.25
+    return device.structured_regular(data), O.Grid.dense(data)
+
+
+def tiled_pair(device):
+    rng = np.random.default_rng(22)
+    k = np.stack(np.meshgrid(*[np.arange(6)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    leaf = k[rng.random(len(k)) < 0.4] * 8
+    tile2 = np.array([[128, 0, 0], [0, 128, 128]])
+    origins = np.concatenate([leaf, tile2, [[4096, 0, 0]]]).astype(np.int32)
+    level = np.array([3] * len(leaf) + [2] * len(tile2) + [1], np.uint32)
+    fmt = np.array([1] * len(leaf) + [0] * (len(tile2) + 1), np.uint32)
+    dense = rng.uniform(0, 1, (len(leaf), 512)).astype(np.float32)
+    dense[rng.random(dense.shape) < 0.002] = np.nan
+    kw = dict(packed_dense=[dense.reshape(-1)], packed_tile=[np.array([0.4, 0.7, 0.2], np.float32)])
+    return device.vdb(level, origins, fmt, **kw), O.Grid.vdb(level, origins, fmt, **kw)
+
+
+def rays(box, count, seed):
+    """Random rays towards the inner 150^3 of the box, and axis-aligned ones,
+    some from integer coordinates."""
+    lo, hi = np.asarray(box[:3]), np.minimum(np.asarray(box[3:]), np.asarray(box[:3]) + 150)
+    org, d = rays_through(np.concatenate([lo, hi]).astype(np.float32), count, seed)
+    rng = np.random.default_rng(seed + 1)
+    for i in range(0, count, 3):
+        axis, sign = rng.integers(3), rng.choice([-1.0, 1.0])
+        o = np.floor(lo + rng.random(3) * (hi - lo)) if i % 2 else lo + rng.random(3) * (hi - lo)
+        o[axis] = (lo if sign > 0 else hi)[axis] - 3.0 * sign
+        org[i], d[i] = o, [0.0, -0.0, 0.0]
+        d[i, axis] = sign
+    return org, d
+
+
+@pytest.mark.parametrize("which", ["dense", "tiled"])
+@pytest.mark.parametrize("count", [1, 65, 400])
+def test_hits(device, which, count):
+    vol, grid = (dense_pair if which == "dense" else tiled_pair)(device)
+    values = [0.25, 0.4, -0.3, 0.41]
+    org, d = rays(grid.bounding_box(), count, 31)
+    tr = np.tile(np.array([[2.3, 77.7]], np.float32), (count, 1))
+    ctx = vol.sampler().hit_context(values)
+    args = [torch.from_numpy(a).cuda() for a in (org, d, tr)]
+    out, cnt = ctx.batch(args[0], args[1], t_ranges=args[2], max_per_ray=48)
+    out, cnt = out.cpu().numpy(), cnt.cpu().numpy()
+    for r in range(count):
+        want = grid.hits(org[r], d[r], values, t_range=tr[r], max_out=48)
+        assert cnt[r] == len(want), r
+        np.testing.assert_array_equal(out[r, :cnt[r]].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("which", ["dense", "tiled"])
+@pytest.mark.parametrize("hint", [0.0, 0.25, 0.5, 1.0])
+@pytest.mark.parametrize("ranges", [None, [[0.1, 0.2], [0.6, 0.9]]], ids=["all", "selected"])
+def test_intervals(device, which, hint, ranges):
+    vol, grid = (dense_pair if which == "dense" else tiled_pair)(device)
+    org, d = rays(grid.bounding_box(), 130, 33)
+    ctx = vol.sampler().interval_context(hint=hint, value_ranges=ranges)
+    out, cnt = ctx.batch(torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda(), max_per_ray=1024)
+    compare_intervals((out.cpu().numpy(), cnt.cpu().numpy()), grid, org, d, O.map_depth(hint), value_ranges=ranges,
+                      max_per_ray=1024)
