@@ -576,10 +576,33 @@ struct TemporalDenseSource
     return voxel(((uint64_t)oz * ny + oy) * nx + ox);
   }
 
-  // A rolled loop: one inlined copy of the time interpolation per stencil
-  // instead of eight.
+  // Structured time steps, stencil inside the domain: the step and weight are
+  // the same for every voxel, so the 8 corners are 8 independent loads of two
+  // neighbouring steps each (temporallyStructured's arithmetic). Otherwise a
+  // rolled loop: one inlined copy of the time interpolation per stencil
+  // instead of eight. 2^20 random points at random times in 160 x 144 x 131
+  // floats of 4 steps: 157 -> 95 us (117 us with the x neighbours four loads
+  // apart, when the second one is fetched again).
   VKL_DEV void corners8(I3 ic, float *s) const
   {
+    const uint32_t ox = (uint32_t)(ic.x - rx), oy = (uint32_t)(ic.y - ry), oz = (uint32_t)(ic.z - rz);
+    if (format == 1u && numTimesteps > 1u && ox < nx - 1u && oy < ny - 1u && oz < nz - 1u) {
+      const float tf       = vmin(vmax(time, 0.f), 1.f) * (float)(numTimesteps - 1u);
+      const uint32_t ts    = (uint32_t)tf;
+      const float w        = tf - (float)ts;
+      const uint32_t next  = (w == 0.f) ? ts : ts + 1u;
+      const uint32_t first = ts < numTimesteps - 2u ? ts : numTimesteps - 2u;  // both steps are in the pair from here
+      const uint64_t v     = ((uint64_t)oz * ny + oy) * nx + ox;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int i       = (k >> 1) | ((k & 1) << 2);  // x neighbours, mostly one cache line, in turn
+        const uint64_t vi = v + ((i & 1) ? (uint64_t)nx * ny : 0u) + ((i & 2) ? nx : 0u) + ((i & 4) ? 1u : 0u);
+        const VoxelRow<T, 2> r = loadRow<T, 2>(data + (vi * numTimesteps + first), 0);
+        const float a = toFloat(r.v[0]), b = toFloat(r.v[1]);
+        s[i] = (1.f - w) * (ts == first ? a : b) + w * (next == first ? a : b);
+      }
+      return;
+    }
 #pragma unroll 1
     for (int i = 0; i < 8; i++) s[i] = at(ic.x + ((i >> 2) & 1), ic.y + ((i >> 1) & 1), ic.z + (i & 1));
   }

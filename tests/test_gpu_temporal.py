@@ -258,3 +258,30 @@ def test_vdb_temporal_observer_and_errors(device):
                                             corner_packed=True),
                  "cornerPacked is not supported for temporal data")
     assert n > 100
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.int16, np.float16, np.float32, np.float64])
+@pytest.mark.parametrize("steps", [1, 2, 3, 7])
+def test_structured_step_pairs(device, dtype, steps):
+    """Linear samples read two neighbouring steps per voxel: times on, between
+    and at the ends of the steps, stencils inside, on the faces and outside, the
+    smallest volume that has a whole stencil."""
+    rng = np.random.default_rng(steps)
+    for dims in ((2, 2, 2), (9, 5, 7)):
+        data = rng.uniform(0, 200, dims[0] * dims[1] * dims[2] * steps).astype(dtype)
+        vol = device.structured_regular(data, dims=dims, structured_steps=steps)
+        grid = O.Grid.dense_temporal(dims, data, structured_steps=steps)
+        hi = np.array(dims, np.float32) - 1
+        pts = np.concatenate([V.uniform_points(1500, (0, 0, 0), hi), V.uniform_points(300, (-1.5, -1.5, -1.5), hi + 1.5),
+                              rng.integers(0, 9, (200, 3)).astype(np.float32)]).astype(np.float32)
+        times = rng.random(len(pts)).astype(np.float32)
+        times[::5] = rng.integers(0, steps, len(times[::5])) / np.float32(max(steps - 1, 1))
+        times[::11], times[1::11] = 0.0, 1.0
+        s = vol.sampler(filter=vkl.VKL_FILTER_LINEAR)
+        grid.set_sampler(O.LINEAR)
+        d, t = torch.from_numpy(pts).cuda(), torch.from_numpy(times).cuda()
+        got, want = s.sample(d, times=t).cpu().numpy(), grid.sample(pts, times=times)
+        same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+        assert same.all(), (dims, np.argmin(same))
+        g, w = s.gradient(d, times=t).cpu().numpy(), grid.gradient(pts, times=times)
+        assert ((g.view(np.uint32) == w.view(np.uint32)) | (np.isnan(g) & np.isnan(w))).all(), dims
