@@ -56,3 +56,25 @@ def test_leaf_rows(device, dtype):
     grid.set_sampler(O.LINEAR)
     assert_same(s.sample(d).cpu().numpy(), grid.sample(pts))
     assert_same(s.gradient(d).cpu().numpy(), grid.gradient(pts))
+
+
+def test_cell_of_special_coordinates(device):
+    """Cells of coordinates where float -> int conversion is special: signed
+    zeros and subnormals, halves, integers, the ends of the int range, infinities
+    and NaN."""
+    big = [2.0 ** 31, -2.0 ** 31, 2147483520.0, -2147483904.0, 3e38, -3e38, np.inf, -np.inf, np.nan]
+    small = [0.0, -0.0, 1e-45, -1e-45, 1.2e-38, -1.2e-38, 0.5, -0.5, 1.0, -1.0, 0.99999994, -0.99999994, 2.5, 6.0]
+    axis = np.array(big + small, np.float32)
+    data = np.random.default_rng(3).uniform(-1, 1, (7, 7, 7)).astype(np.float32)
+    kw = dict(origin=(0, 0, 0), background=5.0)
+    vol, grid = device.structured_regular(data, **kw), O.Grid.dense(data, **kw)
+    pts = np.full((3 * len(axis) + len(axis) ** 2, 3), 2.25, np.float32)
+    for a in range(3):
+        pts[a * len(axis):(a + 1) * len(axis), a] = axis
+    pts[3 * len(axis):, 0], pts[3 * len(axis):, 2] = np.repeat(axis, len(axis)), np.tile(axis, len(axis))
+    d = torch.from_numpy(pts).cuda()
+    for filt, ofilt in ((vkl.VKL_FILTER_NEAREST, O.NEAREST), (vkl.VKL_FILTER_LINEAR, O.LINEAR)):
+        s = vol.sampler(filter=filt)
+        grid.set_sampler(ofilt)
+        assert_same(s.sample(d).cpu().numpy(), grid.sample(pts))
+    assert_same(s.gradient(d).cpu().numpy(), grid.gradient(pts))
