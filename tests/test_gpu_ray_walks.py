@@ -79,3 +79,30 @@ def test_intervals(device, which, hint, ranges):
     out, cnt = ctx.batch(torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda(), max_per_ray=1024)
     compare_intervals((out.cpu().numpy(), cnt.cpu().numpy()), grid, org, d, O.map_depth(hint), value_ranges=ranges,
                       max_per_ray=1024)
+
+
+@pytest.mark.parametrize("which", ["dense", "tiled"])
+@pytest.mark.parametrize("entries", [1, 2, 256, 257, 1024, 1025])
+def test_transfer_function_sizes(device, which, entries):
+    """Interval rendering and Woodcock tracking with tables on both sides of
+    the sizes that are staged in LDS."""
+    vol, grid = (dense_pair if which == "dense" else tiled_pair)(device)
+    org, d = rays(grid.bounding_box(), 200, 35)
+    tf = np.random.default_rng(entries).random((entries, 4), dtype=np.float32)
+    tf[:, 3] *= 0.2
+    rng = (-0.5, 1.25)
+    s = vol.sampler()
+    grid.set_sampler(O.LINEAR)
+    o, dd, t = (torch.from_numpy(a).cuda() for a in (org, d, tf))
+    got, cnt = s.interval_context().ray_march(o, dd, t, rng)
+    want, wcnt = grid.ray_march_intervals(org, d, tf, rng)
+    np.testing.assert_array_equal(cnt.cpu().numpy().view(np.uint32), wcnt)
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    tr = np.tile(np.array([[0.0, 120.0]], np.float32), (200, 1))
+    state = np.stack([np.full(200, 7, np.uint32), np.arange(200, dtype=np.uint32)], 1)
+    ev, sm, n = s.woodcock(o, dd, torch.from_numpy(tr).cuda(), torch.from_numpy(state.view(np.int32)).cuda(), 0.5, t, rng)
+    wev, wsm, wn = grid.woodcock(org, d, tr, state.copy(), 0.5, tf, rng)[:3]
+    for a, b in ((ev, wev), (sm, wsm)):
+        a, b = a.cpu().numpy(), np.asarray(b, np.float32)
+        assert ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
+    np.testing.assert_array_equal(n.cpu().numpy().view(np.uint32), np.asarray(wn, np.uint32))
