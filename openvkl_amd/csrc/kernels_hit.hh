@@ -112,7 +112,7 @@ __global__ __launch_bounds__(1) void kHitNext(const IteratorContextView *__restr
 // Bound by dependent loads (query, index, leaf) and by lanes that wait for
 // each other, so every lane advances by one tick of its search per pass:
 // 2^17 incoherent rays in a 1024^3 half vdb 15.2 -> 5.7 ms against nested
-// loops per ray (8.6 instead of 3.3 lanes active). 4 waves per SIMD (105
+// loops per ray (5.4 with part-filled wavefronts and typed query reads) (8.6 instead of 3.3 lanes active). 4 waves per SIMD (105
 // VGPRs on vdb sources, no spill); cubic filters keep the compiler's choice.
 template <typename Src, int kFilter, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : 4)))

@@ -40,8 +40,8 @@ constexpr uint32_t kShadeVote = 16;
 // query, and in registers they displaced the search's own state.
 //
 // Bound by instruction issue with part of the lanes idle: a 1080p frame of a
-// 300 x 260 x 340 float volume with two iso values 31-33 -> 21-22 ms against
-// nested loops per query (22 instead of 9 lanes active, 212 k instead of
+// 300 x 260 x 340 float volume with two iso values 31.2 -> 21.0 ms against
+// nested loops per query (19.1 since its queries read typed memory) (22 instead of 9 lanes active, 212 k instead of
 // 538 k vector instructions a wavefront). 3 waves per SIMD (168 VGPRs): 2
 // waves 30 ms; 4 and more spill the search's state, 40-80 ms. Shading when
 // 12 to 28 lanes wait measured the same; waiting for all 64 took 7 % longer.
