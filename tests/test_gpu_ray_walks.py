@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+import openvkl_amd as vkl
 from tests import volumes as V
 from tests.test_gpu_iterators import compare_intervals, rays_through
 
@@ -106,3 +107,40 @@ def test_transfer_function_sizes(device, which, entries):
         a, b = a.cpu().numpy(), np.asarray(b, np.float32)
         assert ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
     np.testing.assert_array_equal(n.cpu().numpy().view(np.uint32), np.asarray(wn, np.uint32))
+
+
+def far_rays(box, count, seed):
+    """Rays from 150 voxels away through the inside of the box, so that the
+    walk's accumulated t differs from the box exit's on many of them."""
+    rng = np.random.default_rng(seed)
+    lo, hi = np.asarray(box[:3], np.float64), np.asarray(box[3:], np.float64)
+    out = rng.standard_normal((count, 3))
+    org = (lo + hi) / 2 + 150.0 * out / np.linalg.norm(out, axis=1, keepdims=True)
+    d = lo + rng.random((count, 3)) * (hi - lo) - org
+    return org.astype(np.float32), (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+
+
+@pytest.mark.parametrize("dims", [(45, 38, 51), (9, 64, 23), (40, 48, 33)])
+@pytest.mark.parametrize("cell_centered", [True, False])
+def test_intervals_end_at_the_upper_faces(device, dims, cell_centered):
+    """Every voxel an interval, upper faces inside an 8^3 block: a walk that
+    steps over one has left the volume, in the batch, the plan and the per-ray
+    calls."""
+    data = np.random.default_rng(41).uniform(0, 1, dims[::-1]).astype(np.float32)
+    vol = device.structured_regular(data, cell_centered=cell_centered)
+    grid = O.Grid.dense(data, cell_centered=cell_centered)
+    org, d = far_rays(grid.bounding_box(), 1000, 42)
+    ctx = vol.sampler().interval_context(hint=1.0)
+    o, dd = torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda()
+    out, cnt = (a.cpu().numpy() for a in ctx.batch(o, dd, max_per_ray=256))
+    compare_intervals((out, cnt), grid, org, d, O.map_depth(1.0), max_per_ray=256)
+    plan = vkl.RayBatchPlan(device, [(ctx, o, dd, 256)])
+    plan.execute()
+    torch.cuda.synchronize()
+    res, n = plan.results[0].cpu().numpy(), plan.counts[0].cpu().numpy()
+    plan.release()
+    np.testing.assert_array_equal(n, cnt)
+    for r in range(len(org)):
+        np.testing.assert_array_equal(res[r, :n[r]].view(np.uint32), out[r, :n[r]].view(np.uint32))
+    for r in range(0, len(org), 125):
+        np.testing.assert_array_equal(ctx.intervals(org[r], d[r]).view(np.uint32), out[r, :cnt[r]].view(np.uint32))
