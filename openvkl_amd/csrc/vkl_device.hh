@@ -1361,12 +1361,6 @@ VKL_DEV void queryVoxel(const IteratorContextView &c, int32_t x, int32_t y, int3
   }
   (void)queryLevel<2>(c, x, y, z, depth, desc, node);
 }
-
-VKL_DEV bool inActive(const GridView &g, int32_t x, int32_t y, int32_t z)
-{
-  return (uint32_t)x < g.activeSize[0] && (uint32_t)y < g.activeSize[1] && (uint32_t)z < g.activeSize[2];
-}
-
 // VdbQueryVoxelDense.ih:115-164 (nodes numbered x-fastest, one level-1 node).
 VKL_DEV void queryVoxelDense(const IteratorContextView &c, int32_t x, int32_t y, int32_t z, uint32_t depth,
                              VoxelDesc &desc)
@@ -1374,7 +1368,7 @@ VKL_DEV void queryVoxelDense(const IteratorContextView &c, int32_t x, int32_t y,
   const GridView &g = c.sampler.grid;
   desc.level        = depth;
   const uint32_t ox = (uint32_t)x, oy = (uint32_t)y, oz = (uint32_t)z;
-  if (!inActive(g, x, y, z)) {
+  if (!(ox < g.activeSize[0] && oy < g.activeSize[1] && oz < g.activeSize[2])) {
     desc.isEmpty = true;
     return;
   }
@@ -1466,12 +1460,11 @@ VKL_DEV int intervalTick(const IteratorContextView &c, IntervalState &it, Interv
   // Every step advances t by a positive tDelta; a ray whose steps make no
   // progress (infinite direction components) is ended after kMaxDdaSteps.
   if (!(dda.t <= it.tMax) || ++w.steps > kMaxDdaSteps) return 2;
-  const I3 cell    = ddaCell<kDepth>(dda);
-  const bool dense = kQuery >= 0 ? kQuery == 1 : denseQuery(c.sampler.grid);
+  const I3 cell = ddaCell<kDepth>(dda);
   VoxelDesc v{3u, false, w.leafRange};
   if (kDepth != 3 || !w.inLeaf) {
     const uint32_t l = ddaLevel<kDepth>(dda);
-    if (dense)
+    if (kQuery >= 0 ? kQuery == 1 : denseQuery(c.sampler.grid))
       queryVoxelDense(c, cell.x, cell.y, cell.z, l, v);
     else
       queryVoxel<kNodeCache>(c, cell.x, cell.y, cell.z, l, v, it);
@@ -1484,8 +1477,11 @@ VKL_DEV int intervalTick(const IteratorContextView &c, IntervalState &it, Interv
     // may cut a leaf: there the next cell has to lie inside, too.
     const I3 to = ddaCell<kDepth>(dda);
     w.inLeaf    = !v.isEmpty && v.level == 3u &&
-               (uint32_t)((cell.x ^ to.x) | (cell.y ^ to.y) | (cell.z ^ to.z)) < kRes[3] &&
-               (!dense || inActive(c.sampler.grid, to.x, to.y, to.z));
+               (uint32_t)((cell.x ^ to.x) | (cell.y ^ to.y) | (cell.z ^ to.z)) < kRes[3];
+    if (kQuery >= 0 ? kQuery == 1 : denseQuery(c.sampler.grid)) {
+      const uint32_t *n = c.sampler.grid.activeSize;
+      w.inLeaf          = w.inLeaf && (uint32_t)to.x < n[0] && (uint32_t)to.y < n[1] && (uint32_t)to.z < n[2];
+    }
     w.leafRange = v.valueRange;
   }
   if (v.isEmpty) return 0;
