@@ -144,3 +144,20 @@ def test_intervals_end_at_the_upper_faces(device, dims, cell_centered):
         np.testing.assert_array_equal(res[r, :n[r]].view(np.uint32), out[r, :n[r]].view(np.uint32))
     for r in range(0, len(org), 125):
         np.testing.assert_array_equal(ctx.intervals(org[r], d[r]).view(np.uint32), out[r, :cnt[r]].view(np.uint32))
+
+
+@pytest.mark.parametrize("which", ["dense", "tiled"])
+@pytest.mark.parametrize("hint", [0.5, 1.0])
+@pytest.mark.parametrize("count", [1, 2, 3, 9, 40])
+def test_many_value_ranges(device, which, hint, count):
+    """Selectors of one to many ranges, in any order, overlapping ones among
+    them, values below, between and above all of them."""
+    vol, grid = (dense_pair if which == "dense" else tiled_pair)(device)
+    rng = np.random.default_rng(43 + count)
+    lo = rng.uniform(0.05, 0.8, count)
+    ranges = np.stack([lo, lo + rng.uniform(0.001, 0.03, count)], 1).astype(np.float32)
+    org, d = rays(grid.bounding_box(), 130, 44)
+    ctx = vol.sampler().interval_context(hint=hint, value_ranges=ranges)
+    out, cnt = ctx.batch(torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda(), max_per_ray=1024)
+    compare_intervals((out.cpu().numpy(), cnt.cpu().numpy()), grid, org, d, O.map_depth(hint), value_ranges=ranges,
+                      max_per_ray=1024)
