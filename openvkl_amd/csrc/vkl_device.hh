@@ -949,12 +949,29 @@ VKL_DEV F3 gradientCubic(const Src &src, F3 p)
   return cubicGradientFromTaps(S, p, ic);
 }
 
-// gradientCubic with one x slice of the stencil (16 taps) alive at a time:
-// the same sums in the same order. For kernels that keep much state of their
-// own across the call, where 64 live taps would push that state to scratch.
+// Whether a source's voxels are plain loads, which a stencil can hold many of;
+// a vdb or temporal voxel is a search of its own.
+template <typename Src>
+struct PlainVoxels : std::false_type
+{
+};
+template <typename T, bool kIdx64>
+struct PlainVoxels<DenseSource<T, kIdx64>> : std::true_type
+{
+};
+
+// gradientCubic with one x slice of the stencil (16 taps) alive at a time, or
+// on vdb and temporal sources one tap: the same sums in the same order. For
+// kernels that keep much state of their own across the call, where 64 live
+// taps would push that state to scratch. 16 unrolled searches of a vdb do that
+// as well, whether the call is reached or not (300 bytes a lane of the hit
+// renderer, now 36): 1080p hit rendering of a 512^3 float shell with linear
+// gradients 145 -> 49 ms. Plain voxels keep the slices: 6.5 ms a 960 x 540
+// image with tricubic normals against 8.4 tap by tap.
 template <typename Src>
 VKL_DEV F3 gradientCubicBySlices(const Src &src, F3 p)
 {
+  constexpr int kUnroll = PlainVoxels<Src>::value ? 4 : 1;
   const I3 ic = {floorToInt(p.x), floorToInt(p.y), floorToInt(p.z)};
   const F3 d  = {p.x - (float)ic.x, p.y - (float)ic.y, p.z - (float)ic.z};
   float wx[4], wy[4], wz[4], dx[4], dy[4], dz[4];
@@ -964,26 +981,27 @@ VKL_DEV F3 gradientCubicBySlices(const Src &src, F3 p)
   crDerivWeights(d.x, dx);
   crDerivWeights(d.y, dy);
   crDerivWeights(d.z, dz);
+  const auto pick = [](const float *w, int i) { return i == 0 ? w[0] : i == 1 ? w[1] : i == 2 ? w[2] : w[3]; };
   F3 g = {0.f, 0.f, 0.f};
 #pragma unroll 1
   for (int i = 0; i < 4; i++) {
-    const float wi = i == 0 ? wx[0] : i == 1 ? wx[1] : i == 2 ? wx[2] : wx[3];
-    const float di = i == 0 ? dx[0] : i == 1 ? dx[1] : i == 2 ? dx[2] : dx[3];
     float gy_v = 0.f, gy_dy = 0.f, gy_dz = 0.f;
-#pragma unroll
+#pragma unroll kUnroll
     for (int j = 0; j < 4; j++) {
-      float q[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) q[k] = src.at(ic.x + i - 1, ic.y + j - 1, ic.z + k - 1);
-      const float vz  = wz[0] * q[0] + wz[1] * q[1] + wz[2] * q[2] + wz[3] * q[3];
-      const float dzv = dz[0] * q[0] + dz[1] * q[1] + dz[2] * q[2] + dz[3] * q[3];
-      gy_v += wy[j] * vz;
-      gy_dy += dy[j] * vz;
-      gy_dz += wy[j] * dzv;
+      float vz = 0.f, dzv = 0.f;
+#pragma unroll kUnroll
+      for (int k = 0; k < 4; k++) {
+        const float q = src.at(ic.x + i - 1, ic.y + j - 1, ic.z + k - 1);
+        vz            = k ? vz + pick(wz, k) * q : pick(wz, k) * q;
+        dzv           = k ? dzv + pick(dz, k) * q : pick(dz, k) * q;
+      }
+      gy_v += pick(wy, j) * vz;
+      gy_dy += pick(dy, j) * vz;
+      gy_dz += pick(wy, j) * dzv;
     }
-    g.x += di * gy_v;
-    g.y += wi * gy_dy;
-    g.z += wi * gy_dz;
+    g.x += pick(dx, i) * gy_v;
+    g.y += pick(wx, i) * gy_dy;
+    g.z += pick(wx, i) * gy_dz;
   }
   return g;
 }

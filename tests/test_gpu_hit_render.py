@@ -103,3 +103,40 @@ def test_temporal_and_device_pointers(device):
     assert_same(out.cpu().numpy(), want)
     np.testing.assert_array_equal(cnt.cpu().numpy().view(np.uint32), wcnt)
     compare(ctx, grid, org[:0], d[:0], [0.3], tf, (-3.0, 3.0))
+
+
+def cubic_gradient_pair(device, which):
+    if which == "vdb":
+        origins, leaves = V.sparse_shell_leaves(res=64)
+        n = len(origins)
+        lv, fm = np.full(n, 3, np.uint32), np.full(n, vkl.VKL_FORMAT_DENSE_ZYX, np.uint32)
+        return device.vdb(lv, origins, fm, packed_dense=[leaves.reshape(-1)]), \
+            O.Grid.vdb(lv, origins, fm, packed_dense=[leaves.reshape(-1)]), [0.5], (0.0, 1.2)
+    dims, spacing = (40, 36, 44), (0.25, 0.3, 0.2)
+    if which == "temporal":
+        data, kw = V.temporal_volume(dims, V.wavelet_time, ("structured", 3), spacing=spacing)
+        return device.structured_regular(data, dims=dims, spacing=spacing, **kw), \
+            O.Grid.dense_temporal(dims, data, spacing=spacing, **kw), [-1.0, 0.5, 1.5], (-3.0, 3.0)
+    data = V.procedural(dims, V.wavelet, spacing=spacing)
+    kw = {"packed": {"corner_packed": True}, "bricks": {"brick_shift": (2, 2, 2)}}.get(which, {})
+    return device.structured_regular(data, spacing=spacing, **kw), O.Grid.dense(data, spacing=spacing), \
+        [-1.0, 0.5, 1.5], (-3.0, 3.0)
+
+
+@pytest.mark.parametrize("which", ["x-fastest", "packed", "bricks", "vdb", "temporal"])
+def test_cubic_gradient_close(device, which):
+    """Tricubic normals under linear hits. The hits, and so the counts and the
+    opacity, are the oracle's. A gradient is within 1e-5 of the field's scale
+    (test_gpu_dense.py); a colour then moves by 1e-4 at most, except where the
+    gradient is too small to have a direction or a light grazes the surface."""
+    vol, grid, iso, tf_range = cubic_gradient_pair(device, which)
+    grid.set_sampler(O.LINEAR, gradient_filter=O.CUBIC)
+    grid.set_cubic_double(True)
+    ctx = vol.sampler(filter=vkl.VKL_FILTER_LINEAR, gradient_filter=vkl.VKL_FILTER_CUBIC).hit_context(iso)
+    org, d = rays_through(grid.bounding_box(), 2037, 36)
+    out, cnt = ctx.render_hits(org, d, tf_table(), tf_range)
+    want, wcnt = grid.hit_render(org, d, iso, tf_table(), tf_range)
+    np.testing.assert_array_equal(cnt, wcnt)
+    assert_same(out[:, 3], want[:, 3])
+    close = (np.abs(out - want) <= 1e-4).all(1)
+    assert (cnt > 0).sum() > 500 and close[cnt > 0].mean() >= 0.99
