@@ -161,3 +161,33 @@ def test_many_value_ranges(device, which, hint, count):
     out, cnt = ctx.batch(torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda(), max_per_ray=1024)
     compare_intervals((out.cpu().numpy(), cnt.cpu().numpy()), grid, org, d, O.map_depth(hint), value_ranges=ranges,
                       max_per_ray=1024)
+
+
+@pytest.mark.parametrize("missing", [300, 520])
+def test_tables_beside_rays_that_miss(device, missing):
+    """Whole wavefronts and workgroups whose rays all miss, which do not stage
+    the table, before ones that do, and part-filled last ones."""
+    vol, grid = dense_pair(device)
+    org, d = rays(grid.bounding_box(), missing + 200, 45)
+    d[:missing] = -d[:missing]
+    tf = np.random.default_rng(46).random((64, 4), dtype=np.float32)
+    tf[:, 3] *= 0.2
+    rng = (-0.5, 1.25)
+    s = vol.sampler()
+    grid.set_sampler(O.LINEAR)
+    o, dd, t = (torch.from_numpy(a).cuda() for a in (org, d, tf))
+    got, cnt = s.interval_context().ray_march(o, dd, t, rng)
+    want, wcnt = grid.ray_march_intervals(org, d, tf, rng)
+    assert (wcnt[:missing] == 0).mean() > 0.9 and wcnt[missing:].max() > 0
+    np.testing.assert_array_equal(cnt.cpu().numpy().view(np.uint32), wcnt)
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    n = len(org)
+    tr = np.tile(np.array([[0.0, 120.0]], np.float32), (n, 1))
+    tr[:missing] = [1.0, 0.0]
+    state = np.stack([np.full(n, 7, np.uint32), np.arange(n, dtype=np.uint32)], 1)
+    ev, sm, k = s.woodcock(o, dd, torch.from_numpy(tr).cuda(), torch.from_numpy(state.view(np.int32)).cuda(), 0.5, t, rng)
+    wev, wsm, wk = grid.woodcock(org, d, tr, state.copy(), 0.5, tf, rng)[:3]
+    for a, b in ((ev, wev), (sm, wsm)):
+        a, b = a.cpu().numpy(), np.asarray(b, np.float32)
+        assert ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
+    np.testing.assert_array_equal(k.cpu().numpy().view(np.uint32), np.asarray(wk, np.uint32))
