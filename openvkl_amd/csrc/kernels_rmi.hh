@@ -68,16 +68,25 @@ constexpr uint32_t kTableEntries = 256;
 // rays through a 1024^3 shell, camera / random: 6.26 / 6.23 -> 3.33 / 4.17 ms
 // at depth 2, 14.3 / 19.6 -> 5.3 / 5.9 ms at depth 3, against nested loops
 // per interval; 4 waves per SIMD (5 waves: 15-60 % slower; the compiler's 3
-// at depth 3: 9.2 ms for random rays).
+// at depth 3: 9.2 ms for random rays). At depths 0 and 1 an interval is 128
+// voxels and more, and a lane takes all of its samples before the next one,
+// which keeps camera rays in step: 960 x 540 in a 512^3 float shell at depth
+// 1, 2.60 ms against 3.07 in the one loop (depth 0: the same). Tricubic
+// samples keep the one loop there (480 x 270: 8.4 against 9.7 ms).
 //
 // structuredRegular sources: bound by instruction issue on coherent rays,
 // whose lanes share voxel lines as long as they stay in step, which the
 // nested loops keep (one loop as above: 8.0-10.2 ms a 1080p frame of the
 // 512^3 volume against 4.9, which is 3.7 with the steps since). 5 waves per SIMD: 94 VGPRs without spill at
 // depth 2, the default (4 waves the same, 6 waves 7 % slower).
+template <int kFilter, int kDepth>
+constexpr bool wholeIntervals()
+{
+  return kDepth <= 1 && kFilter != kFilterCubic;
+}
 template <typename Src, int kFilter, int kDepth, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((
-    amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : !IsDenseSource<Src>::value ? 4 : 5)))
+    amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : IsDenseSource<Src>::value ? 5 : kDepth <= 1 ? 1 : 4)))
 void kRayMarchIntervals(const IteratorContextView *__restrict__ cp,
                                                                   AttrView a, RayMarchIntervalsArgs m)
 {
@@ -131,17 +140,24 @@ void kRayMarchIntervals(const IteratorContextView *__restrict__ cp,
     IntervalWalk walk;
     float lo = 0.f, hi = 0.f, end = 0.f;  // the next sub-interval, the interval's end
     while (alpha < 0.99f && taken < m.maxSamples) {
-      const uint32_t waiting = (uint32_t)__popcll(__ballot(!(hi - lo > 0.f)));
-      const uint32_t others  = (uint32_t)__popcll(__ballot(hi - lo > 0.f));
-      if (waiting * kMarchIntervalVote >= others) {
-        if (!(hi - lo > 0.f)) {
-          IntervalOut iv;
-          const int event = intervalTick<false, kDepth, kQuery>(c, st, walk, iv);
-          if (event == 2) break;
-          if (event == 1) {
-            lo  = iv.tLower;
-            end = iv.tUpper;
-            hi  = minf_(lo + dtNominal, end);
+      IntervalOut iv;
+      if constexpr (wholeIntervals<kFilter, kDepth>()) {
+        if (!intervalNext<false, kDepth, kQuery>(c, st, iv)) break;
+        lo  = iv.tLower;
+        end = iv.tUpper;
+        hi  = minf_(lo + dtNominal, end);
+      } else {
+        const uint32_t waiting = (uint32_t)__popcll(__ballot(!(hi - lo > 0.f)));
+        const uint32_t others  = (uint32_t)__popcll(__ballot(hi - lo > 0.f));
+        if (waiting * kMarchIntervalVote >= others) {
+          if (!(hi - lo > 0.f)) {
+            const int event = intervalTick<false, kDepth, kQuery>(c, st, walk, iv);
+            if (event == 2) break;
+            if (event == 1) {
+              lo  = iv.tLower;
+              end = iv.tUpper;
+              hi  = minf_(lo + dtNominal, end);
+            }
           }
         }
       }
@@ -150,25 +166,27 @@ void kRayMarchIntervals(const IteratorContextView *__restrict__ cp,
       // at a time), their samples issued together so that the loads overlap,
       // then composited in order with the same stopping rules; samples past
       // a stop are not counted.
-      float tt[kSamplesAhead], dd[kSamplesAhead], ss[kSamplesAhead];
-      uint32_t nk = 0;
+      do {
+        float tt[kSamplesAhead], dd[kSamplesAhead], ss[kSamplesAhead];
+        uint32_t nk = 0;
 #pragma unroll
-      for (int k = 0; k < kSamplesAhead; k++) {
-        const bool live = hi - lo > 0.f;
-        tt[k]           = 0.5f * (lo + hi);
-        dd[k]           = hi - lo;
-        if (live) {
-          nk = k + 1;
-          lo = hi;
-          hi = minf_(lo + dtNominal, end);
+        for (int k = 0; k < kSamplesAhead; k++) {
+          const bool live = hi - lo > 0.f;
+          tt[k]           = 0.5f * (lo + hi);
+          dd[k]           = hi - lo;
+          if (live) {
+            nk = k + 1;
+            lo = hi;
+            hi = minf_(lo + dtNominal, end);
+          }
         }
-      }
 #pragma unroll
-      for (int k = 0; k < kSamplesAhead; k++)
-        ss[k] = (uint32_t)k < nk ? smp(F3{o.x + tt[k] * d.x, o.y + tt[k] * d.y, o.z + tt[k] * d.z}) : 0.f;
+        for (int k = 0; k < kSamplesAhead; k++)
+          ss[k] = (uint32_t)k < nk ? smp(F3{o.x + tt[k] * d.x, o.y + tt[k] * d.y, o.z + tt[k] * d.z}) : 0.f;
 #pragma unroll
-      for (int k = 0; k < kSamplesAhead; k++)
-        if ((uint32_t)k < nk && alpha < 0.99f && taken < m.maxSamples) composite(ss[k], dd[k]);
+        for (int k = 0; k < kSamplesAhead; k++)
+          if ((uint32_t)k < nk && alpha < 0.99f && taken < m.maxSamples) composite(ss[k], dd[k]);
+      } while (wholeIntervals<kFilter, kDepth>() && hi - lo > 0.f && alpha < 0.99f && taken < m.maxSamples);
     }
   }
   m.rgba[4 * r]     = cr;

@@ -121,3 +121,41 @@ def test_device_pointers_ranges_and_cap(wavelet_pair):
     out, cnt = compare(ctx, grid, org, d, tf, (-3.0, 3.0), sampling_rate=4.0, max_samples=5)
     assert cnt.max() == 5
     compare(ctx, grid, org[:0], d[:0], tf, (-3.0, 3.0))
+
+
+@pytest.fixture(scope="module")
+def tiled_vdb(device):
+    """Leaves of noise beside tiles of two levels, so that a ray steps on every
+    level of the node table."""
+    rng = np.random.default_rng(51)
+    k = np.stack(np.meshgrid(*[np.arange(6)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    leaf = k[rng.random(len(k)) < 0.4] * 8
+    origins = np.concatenate([leaf, [[128, 0, 0], [0, 128, 128]]]).astype(np.int32)
+    level = np.array([3] * len(leaf) + [2, 2], np.uint32)
+    fmt = np.array([vkl.VKL_FORMAT_DENSE_ZYX] * len(leaf) + [vkl.VKL_FORMAT_TILE] * 2, np.uint32)
+    kw = dict(packed_dense=[rng.uniform(0, 1, (len(leaf), 512)).astype(np.float32).reshape(-1)],
+              packed_tile=[np.array([0.4, 0.7], np.float32)])
+    return device.vdb(level, origins, fmt, **kw), O.Grid.vdb(level, origins, fmt, **kw)
+
+
+@pytest.mark.parametrize("which", ["dense", "vdb"])
+@pytest.mark.parametrize("hint", [0.0, 0.25, 0.5, 1.0])
+@pytest.mark.parametrize("ranges", [None, [[0.1, 0.3], [0.6, 0.9]]], ids=["all", "selected"])
+def test_every_depth_bitexact(wavelet_pair, tiled_vdb, which, hint, ranges):
+    """Each iterator depth has a kernel of its own: whole and part-filled
+    wavefronts, and a sample cap that ends rays inside an interval."""
+    vol, grid = wavelet_pair if which == "dense" else tiled_vdb
+    grid.set_sampler(O.LINEAR)
+    ctx = vol.sampler().interval_context(hint=hint, value_ranges=ranges)
+    box = grid.bounding_box().copy()
+    box[3:] = np.minimum(box[3:], box[:3] + 150)
+    org, d = rays_through(box, 1000 + 37, 52)
+    tf_range = (-3.0, 3.0) if which == "dense" else (0.0, 1.0)
+    kw = dict(value_ranges=ranges, depth=O.map_depth(hint))
+    for scale, rate, cap in ((0.1, 2.0, 1 << 20), (2.0, 1.0, 1 << 20), (0.05, 2.0, 7)):
+        tf = tf_table(9, 4, scale)
+        out, cnt = ctx.ray_march(org, d, tf, tf_range, sampling_rate=rate, max_samples=cap)
+        want, wcnt = grid.ray_march_intervals(org, d, tf, tf_range, sampling_rate=rate, max_samples=cap, **kw)
+        assert_same(out, want)
+        np.testing.assert_array_equal(cnt, wcnt)
+        assert cnt.max() == 7 if cap == 7 else cnt.max() > 7
