@@ -189,11 +189,15 @@ VKL_DEV void binnedPoint(const GridView &g, const Src &src, F3 p, float noff, ui
   out[i * outStride] = r;
 }
 
+// Two workgroups fit a CU by their bricks (at most 80 KB each), that is 4
+// wavefronts per SIMD. The tricubic ones of float voxels would take 131 VGPRs,
+// for the overflow's row loads, and then only one fits: 2^21 samples of an
+// 1100 x 200 x 180 float volume 361 us, 281 at 128.
 template <typename T, bool kIdx64, int kOp>
-__global__ __launch_bounds__(kSampleBlock) void kBinnedSample(GridView g, AttrView a, BinGeometry b,
-                                                               const float *__restrict__ xyz,
-                                                               float *__restrict__ out, uint32_t outStride,
-                                                               float noff, BinScratch s)
+__global__ __launch_bounds__(kSampleBlock) __attribute__((
+    amdgpu_waves_per_eu(kOp == kBinSampleCubic || kOp == kBinGradientCubic ? 4 : 1)))
+void kBinnedSample(GridView g, AttrView a, BinGeometry b, const float *__restrict__ xyz, float *__restrict__ out,
+                   uint32_t outStride, float noff, BinScratch s)
 {
   extern __shared__ __attribute__((aligned(16))) unsigned char ldsRaw[];
   T *brick = reinterpret_cast<T *>(ldsRaw);
