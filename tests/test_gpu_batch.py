@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import openvkl_amd as vkl
+from tests import volumes as V
 from tests.volumes import leaves_from_dense
 
 pytestmark = pytest.mark.gpu
@@ -113,3 +114,29 @@ def test_batch_plan_many_small_batches(device):
         assert plan.launch_count() == 2
         _check_plan(plan, outs, refs)
         plan.release()
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (4, 4, 4), (5, 7, 6), (33, 3, 9)])
+@pytest.mark.parametrize("merged", [0, 2])
+def test_tricubic_rows(device, dims, merged):
+    """Tricubic batches of every element type on x-fastest volumes, whose
+    stencils are summed row by row, and on the other layouts beside them: the
+    samples of vklComputeSampleN bit for bit, inside, on the faces, outside."""
+    rng = np.random.default_rng(71)
+    field = rng.uniform(0, 100, dims[::-1])
+    samplers, points, want = [], [], []
+    for dtype, kw in [(np.uint8, {}), (np.int16, {}), (np.uint16, {}), (np.float16, {}), (np.float32, {}),
+                      (np.float64, {}), (np.float32, {"brick_shift": (2, 2, 2)}), (np.float16, {"corner_packed": True})]:
+        vol = device.structured_regular(field.astype(dtype), background=37.5, **kw)
+        samplers.append(vol.sampler(filter=vkl.VKL_FILTER_CUBIC))
+        hi = np.array(dims, np.float32) - 1
+        p = np.concatenate([V.uniform_points(1500, (0, 0, 0), hi), V.uniform_points(501, (-2, -2, -2), hi + 2)])
+        points.append(torch.from_numpy(p).cuda())
+        want.append(samplers[-1].sample(points[-1]).cpu().numpy())
+    outs = [torch.zeros(len(p), device="cuda") for p in points]
+    plan = vkl.SampleBatchPlan(device, samplers, points, outs, autotune=merged)
+    plan.execute()
+    torch.cuda.synchronize()
+    plan.release()
+    for got, w in zip(outs, want):
+        np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32), w.view(np.uint32))
