@@ -1812,7 +1812,7 @@ VKL_DEV int hitTick(const IteratorContextView &c, const S &smp, HitSearch &q, Hi
 template <typename S, int kQuery = -1>
 VKL_DEV bool hitNext(const IteratorContextView &c, const S &smp, HitState &h, HitOut &hit)
 {
-  __shared__ float bisect[kBisWords * kHitLanes];
+  float bisect[kBisWords * kHitLanes];  // registers: every index is constant
   HitSearch q;
   q.h = h;
   hitBegin(q, bisect);
