@@ -133,3 +133,45 @@ def test_hit_batch_bitexact(wavelet, shell, which):
         assert got.shape == want.shape, r
         np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
     assert total > 0
+
+
+@pytest.mark.parametrize("which", ["dense", "vdb"])
+def test_cubic_hits_close(wavelet, shell, which):
+    """Hits through the tricubic sample filter. Samples are within 1e-5 of the
+    field's scale of the oracle's, so a hit's t moves by that over the slope
+    along the ray: within 1e-3 of a voxel at all but grazing hits, whose number
+    may differ too."""
+    vol, grid = wavelet if which == "dense" else shell
+    values = [0.5] if which == "vdb" else [0.3, 1.1]
+    voxel = 1.0 if which == "vdb" else 1.0 / 127.0
+    grid.set_sampler(O.CUBIC)
+    grid.set_cubic_double(True)
+    ctx = vol.sampler(filter=vkl.VKL_FILTER_CUBIC).hit_context(values)
+    org, d = rays_through(grid.bounding_box(), 190, seed=124)
+    out, cnt = ctx.batch(torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda(), max_per_ray=64)
+    out, cnt = out.cpu().numpy(), cnt.cpu().numpy()
+    want = [grid.hits(org[r], d[r], values, max_out=64) for r in range(len(org))]
+    grid.set_cubic_double(False)
+    grid.set_sampler(O.LINEAR)
+    same = [r for r in range(len(org)) if cnt[r] == len(want[r])]
+    assert len(same) >= 0.98 * len(org)
+    got, ref = np.concatenate([out[r, :cnt[r]] for r in same]), np.concatenate([want[r] for r in same])
+    close = (np.abs(got[:, 0] - ref[:, 0]) <= 1e-3 * voxel) & (got[:, 1] == ref[:, 1])
+    assert len(ref) > 100 and close.mean() >= 0.98
+
+
+@pytest.mark.parametrize("count", [70_001, 262_144 + 65, 300_000])
+def test_hit_batches_larger_than_the_chip(device, count):
+    """Batches that start part-filled wavefronts, full ones, and more rays than
+    lanes, which the wavefronts then take from the work counter."""
+    rng = np.random.default_rng(61)
+    data = rng.uniform(0, 1, (19, 14, 17)).astype(np.float32)
+    grid = O.Grid.dense(data)
+    ctx = device.structured_regular(data).sampler().hit_context([0.5])
+    org, d = rays_through(grid.bounding_box(), count, seed=62)
+    out, cnt = ctx.batch(torch.from_numpy(org).cuda(), torch.from_numpy(d).cuda(), max_per_ray=4)
+    want, wcnt = grid.iterate_many(org, d, 4, values=[0.5])
+    cnt = cnt.cpu().numpy().view(np.uint32)
+    np.testing.assert_array_equal(cnt, wcnt)
+    live = np.arange(4)[None] < cnt[:, None]
+    np.testing.assert_array_equal(out.cpu().numpy()[live].view(np.uint32), want[live].view(np.uint32))

@@ -78,3 +78,46 @@ def test_cell_of_special_coordinates(device):
         grid.set_sampler(ofilt)
         assert_same(s.sample(d).cpu().numpy(), grid.sample(pts))
     assert_same(s.gradient(d).cpu().numpy(), grid.gradient(pts))
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (4, 4, 4), (5, 7, 6), (33, 3, 9)])
+@pytest.mark.parametrize("background", [float("nan"), 37.5])
+def test_cubic_rows_at_the_faces(device, dims, background):
+    """Tricubic samples and gradients where stencils reach across a face: the
+    background enters there as it does in the oracle, NaN included."""
+    data = np.random.default_rng(13).uniform(0, 100, dims[::-1]).astype(np.float32)
+    vol, grid = device.structured_regular(data, background=background), O.Grid.dense(data, background=background)
+    hi = np.array(dims, np.float32) - 1
+    pts = np.concatenate([V.uniform_points(4000, (0, 0, 0), hi), V.uniform_points(1000, (-2, -2, -2), hi + 2)])
+    d = torch.from_numpy(pts).cuda()
+    s = vol.sampler(filter=vkl.VKL_FILTER_CUBIC, gradient_filter=vkl.VKL_FILTER_CUBIC)
+    grid.set_sampler(O.CUBIC, gradient_filter=O.CUBIC)
+    for gradient in (False, True):
+        got = (s.gradient if gradient else s.sample)(d).cpu().numpy()
+        want = (grid.gradient if gradient else grid.sample)(pts)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        if not np.isnan(want).all():
+            check_cubic(grid, got, pts, gradient=gradient)
+
+
+def test_row_offsets_above_2_gib(device):
+    """Row offsets are 32-bit byte offsets up to 4 GiB: a uint8 volume of just
+    less. The lerps of 8 bytes round 3 times each way, below 255 * 2e-6."""
+    nx, ny, nz = 2048, 2048, 1020
+    data = torch.randint(0, 256, (nz, ny, nx), dtype=torch.uint8, device="cuda:0",
+                         generator=torch.Generator(device="cuda:0").manual_seed(14))
+    vol = device.structured_regular(data)
+    g = torch.Generator(device="cuda:0").manual_seed(15)
+    p = torch.rand((20000, 3), device="cuda:0", generator=g) * torch.tensor([nx - 1.0, ny - 1.0, nz - 1.0], device="cuda:0")
+    p[:5000, 2] = (nz - 1.0) - torch.rand(5000, device="cuda:0", generator=g) * 3.0
+    i = torch.floor(p).long()
+    f = (p - i).double()
+    flat, want = data.reshape(-1), 0.0
+    for c in range(8):
+        k = torch.minimum(i + torch.tensor([c >> 2, (c >> 1) & 1, c & 1], device="cuda:0"),
+                          torch.tensor([nx - 1, ny - 1, nz - 1], device="cuda:0"))
+        w = [f[:, a] if (c >> (2 - a)) & 1 else 1 - f[:, a] for a in range(3)]
+        want = want + w[0] * w[1] * w[2] * flat[(k[:, 2] * ny + k[:, 1]) * nx + k[:, 0]].double()
+    assert int(((i[:, 2] * ny + i[:, 1]) * nx).max()) > 1 << 31
+    got = vol.sampler(filter=vkl.VKL_FILTER_LINEAR).sample(p.contiguous()).double()
+    assert float((got - want).abs().max()) < 1e-3
