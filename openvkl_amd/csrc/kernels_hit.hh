@@ -28,8 +28,8 @@ VKL_DEV Range1f rayRange(const float *tRanges, uint32_t r)
 // The counter starts at the number of launched lanes and only grows; a
 // wavefront ends once the counter has passed numRays and none of its lanes
 // holds a ray. Lanes start on consecutive rays; a batch of fewer rays than
-// lanes is spread evenly over the wavefronts (raysPerWave). Every ray's results are those of the
-// one-ray-per-lane schedule.
+// lanes is spread evenly over the wavefronts (raysPerWave). Every ray's
+// results are those of the one-ray-per-lane schedule.
 constexpr uint32_t kRefill = 16;
 
 // Rays that each of `waves` wavefronts starts with.
@@ -111,8 +111,8 @@ __global__ __launch_bounds__(1) void kHitNext(const IteratorContextView *__restr
 
 // Bound by dependent loads (query, index, leaf) and by lanes that wait for
 // each other, so every lane advances by one tick of its search per pass:
-// 2^17 incoherent rays in a 1024^3 half vdb 15.2 -> 5.7 ms against nested
-// loops per ray (5.4 with part-filled wavefronts and typed query reads) (8.6 instead of 3.3 lanes active). 4 waves per SIMD (105
+// 2^17 incoherent rays in a 1024^3 half vdb 15.1 -> 4.9 ms against nested
+// loops per ray (5.3 instead of 3.3 lanes active). 4 waves per SIMD (105
 // VGPRs on vdb sources, no spill); cubic filters keep the compiler's choice.
 template <typename Src, int kFilter, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : 4)))

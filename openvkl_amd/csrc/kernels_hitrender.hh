@@ -40,11 +40,14 @@ constexpr uint32_t kShadeVote = 16;
 // query, and in registers they displaced the search's own state.
 //
 // Bound by instruction issue with part of the lanes idle: a 1080p frame of a
-// 300 x 260 x 340 float volume with two iso values 31.2 -> 21.0 ms against
-// nested loops per query (19.1 since its queries read typed memory) (22 instead of 9 lanes active, 212 k instead of
-// 538 k vector instructions a wavefront). 3 waves per SIMD (168 VGPRs): 2
-// waves 30 ms; 4 and more spill the search's state, 40-80 ms. Shading when
-// 12 to 28 lanes wait measured the same; waiting for all 64 took 7 % longer.
+// 300 x 260 x 340 float volume with two iso values 33.1 -> 20.2 ms against
+// nested loops per query (22 instead of 9 lanes active, 185 k instead of 538 k
+// vector instructions a wavefront). 3 waves per SIMD (168 VGPRs): 2 waves took
+// 1.4 times as long there, 4 and more spill the search's state and took 2 to 4
+// times. The same line on vdb sources (36 bytes of scratch at 3 waves): 960 x
+// 540 rays in a 512^3 float shell 17.7 ms, 21.1 at 2 waves; a temporal vdb 24.4
+// and 26.9. Shading when 12 to 28 lanes wait measured the same; waiting for all
+// 64 took 7 % longer.
 template <typename Src, int kFilter, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((
     amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : 3)))

@@ -220,10 +220,10 @@ hipError_t launchHitNext(const IteratorContextView &hostView, const IteratorCont
 // Interval batches keep one ray per lane, and each pass of the loop visits
 // one voxel per lane (intervalTick), empty or not, so that a lane never waits
 // for another one's empty stretch: 230 k camera rays through a 1024^3 shell
-// 2.68 -> 0.39 ms against a loop per interval (0.33 with typed query reads). The kernel is specialised on
+// 2.83 -> 0.32 ms against a loop per interval. The kernel is specialised on
 // the context's iterator depth, so the DDA keeps only the levels it walks.
 // Bound by dependent loads, so occupancy pays: 6 waves per SIMD at depth 2
-// (80 VGPRs), 5 at depth 3 (96), both without spill.
+// (78 VGPRs), 5 at depth 3 (96), both without spill.
 template <int kDepth, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((amdgpu_waves_per_eu(kDepth <= 2 ? 6 : 5)))
 void kIntervalBatch(const IteratorContextView *__restrict__ cp, uint32_t numRays,

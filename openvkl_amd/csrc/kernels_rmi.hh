@@ -48,7 +48,9 @@ VKL_DEV float minf_(float a, float b) { return a < b ? a : b; }
 constexpr int kSamplesAhead = 4;
 
 // Lanes of a vdb march that wait for an interval, times this, against the
-// lanes that have samples to take: below it the interval phase waits.
+// lanes that have samples to take: below it the interval phase waits. 960 x
+// 540 rays in a 512^3 float shell, four samples a voxel: 4.09 ms at 3, 4.50 at
+// 1, 4.14 at 2, 4.05 at 6; one sample a voxel 1.53, 1.58, 1.54, 1.55.
 constexpr uint32_t kMarchIntervalVote = 3;
 
 // Transfer functions of up to this many entries are read from LDS (4 KB a
@@ -60,6 +62,14 @@ constexpr uint32_t kMarchIntervalVote = 3;
 // 1.05 ms, 257 1.20 ms; 64 x 48 rays 0.60 and 0.61 ms.
 constexpr uint32_t kTableEntries = 256;
 
+// Whether a vdb march takes an interval's samples to its end before the next
+// interval, instead of mixing both in one loop (below).
+template <int kFilter, int kDepth>
+constexpr bool wholeIntervals()
+{
+  return kDepth <= 1 && kFilter != kFilterCubic;
+}
+
 // rgba[4r..4r+3] = composited colour and accumulated opacity of ray r.
 //
 // vdb sources: bound by dependent loads and by lanes that wait for each
@@ -68,22 +78,25 @@ constexpr uint32_t kTableEntries = 256;
 // rays through a 1024^3 shell, camera / random: 6.26 / 6.23 -> 3.33 / 4.17 ms
 // at depth 2, 14.3 / 19.6 -> 5.3 / 5.9 ms at depth 3, against nested loops
 // per interval; 4 waves per SIMD (5 waves: 15-60 % slower; the compiler's 3
-// at depth 3: 9.2 ms for random rays). At depths 0 and 1 an interval is 128
-// voxels and more, and a lane takes all of its samples before the next one,
-// which keeps camera rays in step: 960 x 540 in a 512^3 float shell at depth
-// 1, 2.60 ms against 3.07 in the one loop (depth 0: the same). Tricubic
-// samples keep the one loop there (480 x 270: 8.4 against 9.7 ms).
+// at depth 3: 9.2 ms for random rays). Observed sources (16-24 B of scratch at
+// depth 3): 960 x 540 in a 512^3 float shell 4.1 -> 3.1 and 13.0 -> 6.2 ms at
+// depths 2 and 3; a temporal vdb (up to 88 B) 6.6 -> 4.7 and 6.9 -> 4.9 ms. At
+// depths 0 and 1 an interval is 128 voxels and more, and a lane takes all of
+// its samples before the next one, which keeps camera rays in step: 960 x 540
+// in a 512^3 float shell at depth 1, 2.60 ms against 3.07 in the one loop
+// (depth 0: the same). Tricubic samples keep the one loop there (480 x 270: 8.4
+// against 9.7 ms).
 //
 // structuredRegular sources: bound by instruction issue on coherent rays,
 // whose lanes share voxel lines as long as they stay in step, which the
-// nested loops keep (one loop as above: 8.0-10.2 ms a 1080p frame of the
-// 512^3 volume against 4.9, which is 3.7 with the steps since). 5 waves per SIMD: 94 VGPRs without spill at
-// depth 2, the default (4 waves the same, 6 waves 7 % slower).
-template <int kFilter, int kDepth>
-constexpr bool wholeIntervals()
-{
-  return kDepth <= 1 && kFilter != kFilterCubic;
-}
+// nested loops keep (one loop as above took twice as long for a 1080p frame of
+// a 512^3 volume, with 5 times the L2 requests). 5 waves per SIMD: 91 VGPRs
+// without spill at depth 2, the default (4 waves the same, 6 waves 7 % slower).
+//
+// Tricubic samples keep the compiler's choice. The row loads of x-fastest
+// volumes cost float voxels a wavefront per SIMD (3 to 2), which bricks pay: 480
+// x 270 rays of 256 x 240 x 220 floats 2.84 -> 1.24 ms x-fastest, 1.43 -> 1.29
+// corner-packed, 2.35 -> 2.58 on bricks. Asking for 3 spills: 1.53, 1.57, 2.71.
 template <typename Src, int kFilter, int kDepth, int kQuery>
 __global__ __launch_bounds__(kIterBlock) __attribute__((
     amdgpu_waves_per_eu(kFilter == kFilterCubic ? 1 : IsDenseSource<Src>::value ? 5 : kDepth <= 1 ? 1 : 4)))
